@@ -342,6 +342,40 @@ int mgb_histogram(const MgbTreeShape* shape, const MgbMatrix* m, const void* bin
 int mgb_predict(const float* X, uint32_t rows, uint32_t cols, const MgbTreeNode* nodes, const uint32_t* tree_offsets,
                 uint32_t trees, float* margin);
 
+/* A tree packed for prediction.  link: bits 0-15 the distance in nodes from a
+ * split node to its left child (the right child follows the left one; 0: a
+ * leaf), bit 16 default_left, bits 17-31 the feature.  word: a leaf's value
+ * (binary32), or a split node's threshold as an order key -- the sign bit of a
+ * number not below 0 flipped, every bit of a negative one, -0 as +0 -- plus
+ * default_left.  A leaf's feature is the model's feature count and its
+ * default_left 1, so that a walk stays there.  Trees follow one another: tree
+ * t is nodes [offsets[t], offsets[t + 1]), children after their parents, both
+ * offsets even (an unused node may fill the end). */
+typedef struct {
+  uint32_t word, link;
+} MgbPackedNode;
+#define MGB_PACKED_FEATURES 32768u  /* packed models have fewer features */
+#define MGB_PACKED_DISTANCE 65535u  /* largest distance to a left child */
+/* Margins (or, for objective 1 = logistic, their sigmoid) of the trees of
+ * offsets[0 .. trees]: out[r] = base[r] (base_value if base is NULL) plus one
+ * leaf a tree, added in tree order.  X: rows x cols floats, or with indptr and
+ * indices a CSR matrix's `entries` values (column indices strictly increasing
+ * within a row; absent entries and NaN follow default_left).  cols is the
+ * model's feature count; depth the deepest tree's.  base may be out. */
+typedef struct {
+  const float* X;
+  const uint64_t* indptr;
+  const uint32_t* indices;
+  const MgbPackedNode* nodes;
+  const uint32_t* offsets;
+  const float* base;
+  float* out;
+  uint64_t entries;
+  uint32_t rows, cols, trees, depth, objective;
+  float base_value;
+} MgbPredict;
+int mgb_predict_packed(const MgbPredict* p);
+
 /* ---- leaf indices and feature contributions -------------------------- *
  * (src/learner.cpp:455-560 Learner::predict types 6 and 2-5.)  Rows are
  * dense (X: rows x cols floats, indptr NULL) or CSR (X holds the values,

@@ -1,0 +1,160 @@
+"""Margin prediction over packed trees against a plain numpy walk of the
+model (value < threshold goes left, NaN and absent entries follow
+default_left; binary32 sums in tree order): bit-identical at the edges of the
+row tiles, for rows too wide for LDS, trees larger than the staged buffer,
+models whose children are not neighbours, and models the packed form does not
+hold."""
+import json
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _random_tree(rng, cols, depth, shuffle):
+    left, right, feat, cond, dleft, level = [-1], [-1], [0], [0.0], [0], [0]
+    k = 0
+    while k < len(left):
+        if level[k] < depth and (level[k] == 0 or rng.random() < 0.93):
+            left[k], right[k] = len(left), len(left) + 1
+            feat[k], dleft[k] = int(rng.integers(cols)), int(rng.integers(2))
+            cond[k] = float(np.float32(rng.normal()))
+            for lst, v in ((left, -1), (right, -1), (feat, 0), (cond, 0.0), (dleft, 0), (level, level[k] + 1)):
+                lst.extend([v, v])
+        else:
+            cond[k] = float(np.float32(rng.normal() * 0.1))
+        k += 1
+    n = len(left)
+    ids = np.arange(n)
+    if shuffle and n > 1:  # a preorder-like numbering: children are not neighbours
+        ids[1:] = 1 + rng.permutation(n - 1)
+    out = {key: [0] * n for key in ("left_children", "right_children", "split_indices", "split_conditions",
+                                    "default_left", "parents", "loss_changes", "sum_hessian", "base_weights")}
+    out["parents"][0] = 2147483647
+    for i in range(n):
+        k = int(ids[i])
+        out["left_children"][k] = int(ids[left[i]]) if left[i] >= 0 else -1
+        out["right_children"][k] = int(ids[right[i]]) if left[i] >= 0 else -1
+        out["split_indices"][k], out["split_conditions"][k] = feat[i], cond[i]
+        out["default_left"][k] = dleft[i]
+        if left[i] >= 0:
+            out["parents"][int(ids[left[i]])] = out["parents"][int(ids[right[i]])] = k
+    return out
+
+
+def _booster(xgb, trees, cols, objective="reg:squarederror"):
+    model = {"version": [3, 5, 0], "learner": {
+        "attributes": {}, "feature_names": [], "feature_types": [],
+        "learner_model_param": {"base_score": "0.25", "num_class": "0", "num_feature": str(cols), "num_target": "1"},
+        "objective": {"name": objective},
+        "gradient_booster": {"name": "gbtree", "model": {"trees": trees, "tree_info": [0] * len(trees)}}}}
+    return xgb.Booster(model_file=bytearray(json.dumps(model).encode()))
+
+
+def _margins(trees, X, base):
+    out = np.broadcast_to(np.asarray(base, np.float32), (len(X),)).copy()
+    rows = np.arange(len(X))
+    for t in trees:
+        left, right = np.array(t["left_children"]), np.array(t["right_children"])
+        feat, cond = np.array(t["split_indices"]), np.array(t["split_conditions"], np.float32)
+        dleft = np.array(t["default_left"])
+        at = np.zeros(len(X), np.int64)
+        while np.any(left[at] >= 0):
+            v = X[rows, feat[at]]
+            go = np.where(np.isnan(v), dleft[at] != 0, v < cond[at])
+            at = np.where(left[at] < 0, at, np.where(go, left[at], right[at]))
+        out = out + cond[at]
+    return out
+
+
+def _values(rng, rows, cols, missing):
+    X = rng.normal(size=(rows, cols)).astype(np.float32)
+    X[rng.random(X.shape) < missing] = np.nan
+    return X
+
+
+@pytest.mark.parametrize("rows,cols,trees,depth,shuffle", [
+    (1, 1, 1, 1, False), (3, 7, 130, 4, True), (64, 32, 65, 6, False), (12287, 5, 3, 3, False),
+    (12288, 31, 9, 5, True), (12289, 64, 70, 8, False), (16384 + 63, 32, 33, 6, False),
+    (70000, 9, 5, 4, False), (81921, 64, 7, 8, False), (13000, 200, 11, 5, False), (12500, 520, 6, 6, False),
+    (12300, 1200, 5, 5, False), (12400, 4, 1100, 2, False), (13000, 6, 2, 13, False), (300, 6, 2, 12, False),
+    (150000, 2, 1, 2, False)])
+def test_margins_equal_plain_walk(xgb, rows, cols, trees, depth, shuffle):
+    rng = np.random.default_rng(rows * 31 + cols)
+    forest = [_random_tree(rng, cols, depth, shuffle) for _ in range(trees)]
+    X = _values(rng, rows, cols, 0.1)
+    bst = _booster(xgb, forest, cols)
+    expect = _margins(forest, X, 0.25)
+    np.testing.assert_array_equal(bst.predict(xgb.DMatrix(X), output_margin=True), expect)
+    np.testing.assert_array_equal(bst.inplace_predict(X), expect)
+    base = rng.normal(size=rows).astype(np.float32)
+    np.testing.assert_array_equal(bst.predict(xgb.DMatrix(X, base_margin=base)), _margins(forest, X, base))
+    if trees > 2:
+        np.testing.assert_array_equal(bst.predict(xgb.DMatrix(X), iteration_range=(1, trees - 1)),
+                                      _margins(forest[1:trees - 1], X, 0.25))
+
+
+@pytest.mark.parametrize("rows,cols,trees,depth,share", [
+    (1, 40, 3, 3, 0.2), (6143, 33, 70, 5, 0.3), (6144, 31, 12, 5, 1.0), (13001, 2000, 20, 6, 0.01),
+    (20000, 64, 9, 8, 0.5), (12500, 30000, 4, 5, 0.002), (300, 33000, 3, 4, 0.01)])
+def test_csr_margins_equal_plain_walk(xgb, rows, cols, trees, depth, share):
+    """Rows of very uneven length, some empty; 33,000 features are past the
+    packed form."""
+    import scipy.sparse as sp
+    rng = np.random.default_rng(rows + cols)
+    used = rng.integers(0, cols, size=min(cols, 60))  # the columns the trees look at
+    forest = [_random_tree(rng, len(used), depth, False) for _ in range(trees)]
+    for t in forest:
+        t["split_indices"] = [int(used[f]) for f in t["split_indices"]]
+    nnz = np.minimum(rng.poisson(share * cols, size=rows), cols)
+    nnz[0] = 0
+    nnz[rows // 2] = min(cols, 4000)
+    indptr = np.concatenate([[0], np.cumsum(nnz)])
+    indices = np.concatenate([np.sort(rng.choice(cols, size=n, replace=False)) for n in nnz]).astype(np.int32)
+    values = rng.normal(size=indptr[-1]).astype(np.float32)
+    values[rng.random(len(values)) < 0.05] = np.nan
+    csr = sp.csr_matrix((values, indices, indptr), shape=(rows, cols))
+    small = np.full((rows, len(used)), np.nan, np.float32)
+    position = {int(c): j for j, c in enumerate(used)}
+    row_of = np.repeat(np.arange(rows), nnz)
+    keep = np.isin(indices, used)
+    small[row_of[keep], [position[int(c)] for c in indices[keep]]] = values[keep]
+    plain = [dict(t, split_indices=[position[f] if l >= 0 else 0 for f, l in
+                                    zip(t["split_indices"], t["left_children"])]) for t in forest]
+    bst = _booster(xgb, forest, cols)
+    np.testing.assert_array_equal(bst.predict(xgb.DMatrix(csr)), _margins(plain, small, 0.25))
+    np.testing.assert_array_equal(bst.inplace_predict(csr), _margins(plain, small, 0.25))
+
+
+def test_trees_added_and_replaced_are_predicted(xgb):
+    """A booster that predicted keeps its packed trees: later rounds join
+    them, and a loaded model takes their place."""
+    rng = np.random.default_rng(3)
+    X = _values(rng, 5000, 8, 0.1)
+    y = np.nan_to_num(X[:, 0] - X[:, 1]).astype(np.float32)
+    d, other = xgb.DMatrix(X, label=y), xgb.DMatrix(X[::-1].copy())
+    params = {"max_depth": 5, "max_bin": 64}
+    bst = xgb.train(params, d, 2)
+    for rounds in (3, 9, 30):
+        bst = xgb.train(params, d, rounds - bst.num_boosted_rounds(), xgb_model=bst)
+        np.testing.assert_array_equal(bst.predict(other)[::-1], bst.predict(d))
+    growing = xgb.Booster(params, [d])
+    for r in range(6):
+        growing.update(d, r)
+        np.testing.assert_array_equal(growing.predict(other)[::-1], growing.predict(d))
+    forest = [_random_tree(rng, 8, 4, False) for _ in range(3)]
+    growing.load_model(_booster(xgb, forest, 8).save_raw())
+    np.testing.assert_array_equal(growing.predict(other), _margins(forest, X[::-1], 0.25))
+
+
+@pytest.mark.parametrize("rows", [7, 13000])
+def test_logistic_output_is_the_sigmoid_of_the_margin(xgb, rows):
+    rng = np.random.default_rng(rows)
+    forest = [_random_tree(rng, 12, 5, False) for _ in range(20)]
+    X = _values(rng, rows, 12, 0.2)
+    bst = _booster(xgb, forest, 12, "binary:logistic")
+    margin = bst.predict(xgb.DMatrix(X), output_margin=True)
+    # Rounding of e^x, two sums and a division: a few units of 2^-24.
+    np.testing.assert_allclose(bst.predict(xgb.DMatrix(X)), 1.0 / (1.0 + np.exp(-margin.astype(np.float64))),
+                               rtol=4e-7, atol=0)

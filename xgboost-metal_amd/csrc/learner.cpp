@@ -507,34 +507,125 @@ void Learner::upload_model() {
   model_version_ = trees.size();
 }
 
-// Adds trees [offsets, offsets + count) of the uploaded model to margin.
-void Learner::predict_into(DMatrix& data, const uint32_t* offsets, uint32_t count, float* margin) {
+namespace {
+
+// Appends a tree in packed form, breadth first (a trained tree's own order);
+// false if it does not fit: a feature or a distance out of range, a NaN
+// threshold, or nodes that are not a tree.
+bool pack_tree(const std::vector<MgbTreeNode>& t, uint32_t features, std::vector<MgbPackedNode>& out,
+               uint32_t& deepest) {
+  std::vector<std::pair<uint32_t, uint32_t>> order;  // (node id, depth) by packed position
+  order.reserve(t.size());
+  if (t.empty()) return false;
+  order.emplace_back(0u, 0u);
+  for (size_t i = 0; i < order.size(); ++i) {
+    const auto [id, depth] = order[i];
+    const MgbTreeNode& n = t[id];
+    MgbPackedNode packed;
+    if (n.left < 0) {
+      std::memcpy(&packed.word, &n.leaf, sizeof(float));
+      packed.link = (features << 17) | (1u << 16);
+    } else {
+      const size_t distance = order.size() - i;
+      if (n.feature < 0 || (uint32_t)n.feature >= features || std::isnan(n.threshold) || distance > MGB_PACKED_DISTANCE ||
+          (size_t)n.left >= t.size() || n.right < 0 || (size_t)n.right >= t.size() || order.size() + 2 > t.size())
+        return false;
+      const float threshold = n.threshold + 0.0f;
+      uint32_t bits;
+      std::memcpy(&bits, &threshold, sizeof(bits));
+      const uint32_t go = n.default_left ? 1u : 0u;
+      packed.word = (bits & 0x80000000u ? ~bits : bits | 0x80000000u) + go;
+      packed.link = (uint32_t)distance | (go << 16) | ((uint32_t)n.feature << 17);
+      order.emplace_back((uint32_t)n.left, depth + 1);
+      order.emplace_back((uint32_t)n.right, depth + 1);
+      deepest = std::max(deepest, depth + 1);
+    }
+    out.push_back(packed);
+  }
+  if (out.size() % 2) out.push_back(MgbPackedNode{0, (features << 17) | (1u << 16)});  // trees start at even nodes
+  return true;
+}
+
+}  // namespace
+
+bool Learner::pack_model() {
+  if (num_feature >= MGB_PACKED_FEATURES) return false;
+  const size_t had = packed_offsets_.size() - 1;
+  while (packed_fits_ && packed_offsets_.size() <= trees.size()) {
+    packed_fits_ = packed_nodes_.size() + trees[packed_offsets_.size() - 1].nodes.size() < UINT32_MAX &&
+                   pack_tree(trees[packed_offsets_.size() - 1].nodes, num_feature, packed_nodes_, packed_depth_);
+    packed_offsets_.push_back((uint32_t)packed_nodes_.size());
+  }
+  if (!packed_fits_) return false;
+  if (packed_offsets_.size() - 1 == had && packed_uploaded_ == packed_nodes_.size()) return true;
+  // New trees follow those on the device; a buffer that is too small is
+  // replaced by one of twice the size and filled again.
+  const size_t bytes = packed_nodes_.size() * sizeof(MgbPackedNode);
+  if (bytes > d_packed_nodes_.bytes()) {
+    packed_uploaded_ = 0;
+    d_packed_nodes_.resize(2 * bytes);
+  }
+  kcheck(mgb_memcpy_h2d_async(d_packed_nodes_.as<MgbPackedNode>() + packed_uploaded_,
+                              packed_nodes_.data() + packed_uploaded_,
+                              (packed_nodes_.size() - packed_uploaded_) * sizeof(MgbPackedNode)),
+         "packed trees upload");
+  const size_t offset_bytes = packed_offsets_.size() * sizeof(uint32_t);
+  if (offset_bytes > d_packed_offsets_.bytes()) d_packed_offsets_.resize(2 * offset_bytes);
+  kcheck(mgb_memcpy_h2d_async(d_packed_offsets_.get(), packed_offsets_.data(), offset_bytes),
+         "packed offsets upload");
+  packed_uploaded_ = packed_nodes_.size();
+  return true;
+}
+
+void Learner::predict_into(DMatrix& data, uint32_t begin, uint32_t end, bool transform, DeviceBuffer& out) {
   data.upload();
-  if (data.sparse)
-    kcheck(mgb_predict_csr(data.d_indptr.as<uint64_t>(), data.d_indices.as<uint32_t>(), data.d_values.as<float>(),
-                           data.rows, d_model_nodes_.as<MgbTreeNode>(), offsets, count, margin),
-           "prediction");
-  else
-    kcheck(mgb_predict(data.d_data.as<float>(), data.rows, data.cols, d_model_nodes_.as<MgbTreeNode>(), offsets,
-                       count, margin),
-           "prediction");
+  out.ensure((size_t)std::max<uint32_t>(data.rows, 1) * sizeof(float));
+  const bool given = !data.base_margin.empty();
+  if (given) {
+    require(data.base_margin.size() == data.rows, "base_margin must have one value per row.");
+    out.upload(data.base_margin.data(), data.rows * sizeof(float));
+  }
+  float* margin = out.as<float>();
+  if (end > begin && pack_model()) {
+    MgbPredict p{};
+    p.X = data.sparse ? data.d_values.as<float>() : data.d_data.as<float>();
+    p.indptr = data.sparse ? data.d_indptr.as<uint64_t>() : nullptr;
+    p.indices = data.sparse ? data.d_indices.as<uint32_t>() : nullptr;
+    p.entries = data.values.size();
+    p.nodes = d_packed_nodes_.as<MgbPackedNode>();
+    p.offsets = d_packed_offsets_.as<uint32_t>() + begin;
+    p.base = given ? margin : nullptr;
+    p.base_value = base_margin_value();
+    p.out = margin;
+    p.rows = data.rows;
+    p.cols = data.cols;
+    p.trees = end - begin;
+    p.depth = packed_depth_;
+    p.objective = transform ? (uint32_t)objective() : 0u;
+    kcheck(mgb_predict_packed(&p), "prediction");
+    return;
+  }
+  // No trees, or a model that the packed form does not hold.
+  if (!given) kcheck(mgb_fill_f32(margin, data.rows, base_margin_value()), "margin fill");
+  if (end > begin) {
+    upload_model();
+    const uint32_t* offsets = d_model_offsets_.as<uint32_t>() + begin;
+    if (data.sparse)
+      kcheck(mgb_predict_csr(data.d_indptr.as<uint64_t>(), data.d_indices.as<uint32_t>(), data.d_values.as<float>(),
+                             data.rows, d_model_nodes_.as<MgbTreeNode>(), offsets, end - begin, margin),
+             "prediction");
+    else
+      kcheck(mgb_predict(data.d_data.as<float>(), data.rows, data.cols, d_model_nodes_.as<MgbTreeNode>(), offsets,
+                         end - begin, margin),
+             "prediction");
+  }
+  if (transform) kcheck(mgb_transform(margin, data.rows, (uint32_t)objective()), "transform");
 }
 
 DeviceBuffer* Learner::margin_cache(DMatrix& data) {
   if (cache_id_ == data.id && cache_trees_ == boosted_rounds() && d_margin_.get()) return &d_margin_;
   drain();  // the margin is rebuilt from every tree
-  data.upload();
-  d_margin_.ensure((size_t)data.rows * sizeof(float));
-  if (!data.base_margin.empty()) {
-    require(data.base_margin.size() == data.rows, "base_margin must have one value per row.");
-    d_margin_.upload(data.base_margin.data(), data.rows * sizeof(float));
-  } else {
-    kcheck(mgb_fill_f32(d_margin_.as<float>(), data.rows, base_margin_value()), "margin fill");
-  }
-  if (!trees.empty()) {
-    upload_model();
-    predict_into(data, d_model_offsets_.as<uint32_t>(), (uint32_t)trees.size(), d_margin_.as<float>());
-  }
+  predict_into(data, 0, (uint32_t)trees.size(), false, d_margin_);
   cache_id_ = data.id;
   cache_trees_ = trees.size();
   return &d_margin_;
@@ -1087,17 +1178,8 @@ const float* Learner::predict_device(DMatrix& data, bool output_margin, uint32_t
     if (output_margin || objective() != 1) return d_margin_.as<float>();
     kcheck(mgb_memcpy_d2d(d_out, d_margin_.get(), data.rows * sizeof(float)), "copy");
   } else {
-    data.upload();
-    if (!data.base_margin.empty()) {
-      require(data.base_margin.size() == data.rows, "base_margin must have one value per row.");
-      scratch.upload(data.base_margin.data(), data.rows * sizeof(float));
-    } else {
-      kcheck(mgb_fill_f32(d_out, data.rows, base_margin_value()), "margin fill");
-    }
-    if (end > begin) {
-      upload_model();
-      predict_into(data, d_model_offsets_.as<uint32_t>() + begin, end - begin, d_out);
-    }
+    predict_into(data, begin, end, !output_margin, scratch);
+    return scratch.as<float>();
   }
   if (!output_margin) kcheck(mgb_transform(d_out, data.rows, (uint32_t)objective()), "transform");
   return d_out;
@@ -1416,6 +1498,11 @@ void Learner::load_model(const Json& input) {
   cache_id_ = 0;
   cache_trees_ = 0;
   model_version_ = SIZE_MAX;
+  packed_nodes_.clear();
+  packed_offsets_.assign(1, 0);
+  packed_depth_ = 0;
+  packed_fits_ = true;
+  packed_uploaded_ = 0;
   metrics.clear();  // src/model.cpp:224
   // A loaded model restarts the engine from seed 0 (src/model.cpp:225).
   rng_.seed(0);

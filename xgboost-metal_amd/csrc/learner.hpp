@@ -196,7 +196,12 @@ class Learner {
   float base_margin_value() const;
   void upload_model();
   DeviceBuffer* margin_cache(DMatrix& data);
-  void predict_into(DMatrix& data, const uint32_t* offsets, uint32_t count, float* margin);
+  // Brings the packed copy of the trees up to date (new trees are appended);
+  // false when a tree does not fit the packed form.
+  bool pack_model();
+  // out[r] = the row's base margin plus its leaves of rounds [begin, end),
+  // through the objective's output transform if asked.
+  void predict_into(DMatrix& data, uint32_t begin, uint32_t end, bool transform, DeviceBuffer& out);
 
   std::map<std::string, std::string> params_;
   // Training-matrix prediction cache.
@@ -211,6 +216,14 @@ class Learner {
   size_t means_version_ = SIZE_MAX;
   size_t model_version_ = SIZE_MAX, model_trees_ = 0;
   size_t uploaded_trees_ = 0;
+  // The trees packed for prediction, on the host and (the first
+  // packed_uploaded_ nodes) on the device.
+  std::vector<MgbPackedNode> packed_nodes_;
+  std::vector<uint32_t> packed_offsets_{0};
+  uint32_t packed_depth_ = 0;
+  bool packed_fits_ = true;
+  size_t packed_uploaded_ = 0;
+  DeviceBuffer d_packed_nodes_, d_packed_offsets_;
   std::map<std::string, double> seconds_;
   uint64_t rounds_timed_ = 0;
   uint64_t hist_bytes_ = 0, hist_rows_ = 0, split_bytes_ = 0, partition_bytes_ = 0;
