@@ -401,6 +401,32 @@ int mgb_predict_contribs(const float* X, const uint64_t* indptr, const uint32_t*
                          const uint32_t* tree_offsets, uint32_t trees, uint32_t max_depth, uint32_t approximate,
                          uint32_t interactions, const float* base, float base_value, float* out);
 
+/* Exact contributions from a table of the trees' paths, laid out once a model:
+ * mgb_shap_elements gives the elements of a path record for trees of this
+ * depth (0: deeper than 16), mgb_shap_table_bytes the table's size.
+ * mgb_shap_paths fills it for `count` leaves: leaves[k] the leaf's place in
+ * `nodes`, parents[i] the place of node i's parent times two, plus one where
+ * node i is its left child (-1 for a root).  mgb_predict_shap: out as
+ * mgb_predict_contribs' (rows x (cols + 1), the bias last: base[r], or
+ * base_value if base is NULL, plus root_means[0 .. trees)), rows dense or CSR;
+ * allocates its scratch (at most 256 MB, or one 64-row tile's). */
+typedef struct {
+  const float* X;
+  const uint64_t* indptr;
+  const uint32_t* indices;
+  const uint32_t* table;
+  const float* root_means;
+  const float* base;
+  float* out;
+  uint32_t rows, cols, leaves, elements, trees;
+  float base_value;
+} MgbShap;
+uint32_t mgb_shap_elements(uint32_t depth);
+size_t mgb_shap_table_bytes(uint32_t leaves, uint32_t elements);
+int mgb_shap_paths(const MgbTreeNode* nodes, const int64_t* parents, const uint32_t* leaves, uint32_t count,
+                   uint32_t elements, uint32_t cols, uint32_t* table);
+int mgb_predict_shap(const MgbShap* p);
+
 /* ---- evaluation metrics (src/metrics.cpp:8-159) ------------------------- */
 /* Elementwise metric kinds, numbered as the reference's metric table
  * (src/metrics.cpp:13-16). */

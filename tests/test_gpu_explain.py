@@ -278,3 +278,91 @@ def test_classifier_apply(xgb):
     model = xgb.XGBClassifier(n_estimators=2, max_depth=2, max_bin=16)
     model.fit(X, (y > 0).astype(np.int64))
     np.testing.assert_array_equal(model.apply(X), model.get_booster().predict(xgb.DMatrix(X), pred_leaf=True))
+
+
+def _tree_shap(t, x, cols):
+    """A tree's exact contributions to row x in binary64, by TreeSHAP's own
+    recursion (Lundberg, Erion and Lee 2018, Algorithm 2) over path weights."""
+    phi = np.zeros(cols)
+
+    def extend(path, z, o, f):
+        path = [list(e) for e in path] + [[f, z, o, 1.0 if not path else 0.0]]
+        n = len(path) - 1
+        for i in range(n - 1, -1, -1):
+            path[i + 1][3] += o * path[i][3] * (i + 1) / (n + 1)
+            path[i][3] = z * path[i][3] * (n - i) / (n + 1)
+        return path
+
+    def unwind(path, k):
+        path = [list(e) for e in path]
+        n, z, o = len(path) - 1, path[k][1], path[k][2]
+        nxt = path[n][3]
+        for i in range(n - 1, -1, -1):
+            if o != 0:
+                kept = path[i][3]
+                path[i][3] = nxt * (n + 1) / ((i + 1) * o)
+                nxt = kept - path[i][3] * z * (n - i) / (n + 1)
+            else:
+                path[i][3] = path[i][3] * (n + 1) / (z * (n - i))
+        for i in range(k, n):
+            path[i][:3] = path[i + 1][:3]
+        return path[:-1]
+
+    def visit(k, path, z, o, f):
+        path = extend(path, z, o, f)
+        if t.left[k] < 0:
+            for i in range(1, len(path)):
+                w = sum(e[3] for e in unwind(path, i))
+                phi[path[i][0]] += w * (path[i][2] - path[i][1]) * float(t.cond[k])
+            return
+        hot = t.child(k, x)
+        cold = t.left[k] + t.right[k] - hot
+        in_z, in_o = 1.0, 1.0
+        for i in range(1, len(path)):
+            if path[i][0] == t.feature[k]:
+                in_z, in_o = path[i][1], path[i][2]
+                path = unwind(path, i)
+                break
+        visit(hot, path, in_z * t.cover[hot] / t.cover[k], in_o, t.feature[k])
+        visit(cold, path, in_z * t.cover[cold] / t.cover[k], 0.0, t.feature[k])
+
+    visit(0, [], 1.0, 1.0, -1)
+    return phi
+
+
+@pytest.mark.parametrize("rows,cols,depth,rounds", [
+    (1, 3, 1, 1), (63, 2, 3, 4), (65, 9, 5, 3), (200, 40, 7, 3), (130, 90, 8, 2), (64, 200, 6, 2), (300, 7, 11, 1),
+    (257, 5, 13, 1), (900, 6, 16, 1), (70, 700, 4, 3), (3000, 4, 2, 9)])
+def test_contributions_over_path_lengths_and_widths(xgb, rows, cols, depth, rounds):
+    """Path tables of every element count, sums in LDS and (700 features) in
+    memory, rows on both sides of a 64-row tile; absent entries as NaN, in a
+    dense and a CSR matrix.  Binary32 sums of products against binary64: the
+    error grows with the terms added, within 2e-5 of the margins' scale."""
+    import scipy.sparse as sp
+    rng = np.random.default_rng(rows + cols + depth)
+    train = rng.normal(size=(2000, cols)).astype(np.float32)
+    y = (rng.normal(size=2000) + train[:, 0] * train[:, -1] + train[:, cols // 2]).astype(np.float32)
+    train[rng.random(train.shape) < 0.1] = np.nan
+    bst = xgb.train({"max_depth": depth, "max_bin": 64, "eta": 0.5, "min_child_weight": 1, "lambda": 0.1},
+                    xgb.DMatrix(train, label=y), rounds)
+    X = rng.normal(size=(rows, cols)).astype(np.float32)
+    X[rng.random(X.shape) < 0.2] = np.nan
+    d = xgb.DMatrix(X)
+    exact = bst.predict(d, pred_contribs=True).astype(np.float64)
+    margin = bst.predict(d, output_margin=True).astype(np.float64)
+    scale = max(1.0, np.abs(margin).max())
+    np.testing.assert_allclose(exact.sum(axis=1), margin, rtol=0, atol=2e-5 * scale)
+    trees = _trees(bst)
+    picked = sorted({0, min(rows - 1, 63), min(rows - 1, 64), rows - 1})[:3 if depth < 11 else 1]
+    for i in picked:
+        ref = sum(_tree_shap(t, X[i], cols) for t in trees)
+        np.testing.assert_allclose(exact[i, :-1], ref, rtol=0, atol=2e-5 * scale)
+    r, c = np.nonzero(~np.isnan(X))
+    csr = sp.csr_matrix((X[r, c], (r, c)), shape=X.shape)
+    np.testing.assert_array_equal(bst.predict(xgb.DMatrix(csr), pred_contribs=True), exact.astype(np.float32))
+    # A shorter range of rounds, then the whole model again.
+    if rounds > 1:
+        part = bst.predict(d, pred_contribs=True, iteration_range=(0, 1))
+        np.testing.assert_allclose(part.sum(axis=1), bst.predict(d, output_margin=True, iteration_range=(0, 1)),
+                                   rtol=0, atol=2e-5 * scale)
+        np.testing.assert_array_equal(bst.predict(d, pred_contribs=True), exact.astype(np.float32))

@@ -1211,6 +1211,49 @@ uint32_t node_means(const std::vector<MgbTreeNode>& t, float* means) {
 
 }  // namespace
 
+// The path table of trees [0, end), laid out on the device from the uploaded
+// nodes.
+void Learner::build_paths(uint32_t end) {
+  if (shap_trees_ == end) return;
+  shap_trees_ = SIZE_MAX;
+  std::vector<int64_t> parents;
+  std::vector<uint32_t> leaves;
+  std::vector<float> roots, means;
+  uint32_t deepest = 0;
+  for (uint32_t t = 0; t < end; ++t) {
+    const auto& nodes = trees[t].nodes;
+    means.resize(nodes.size());
+    deepest = std::max(deepest, node_means(nodes, means.data()));
+    roots.push_back(nodes.empty() ? 0.0f : means[0]);
+    const size_t at = parents.size();
+    parents.resize(at + nodes.size(), -1);
+    for (size_t i = 0; i < nodes.size(); ++i) {
+      if (nodes[i].left < 0) continue;
+      parents[at + nodes[i].left] = (int64_t)(at + i) * 2 + 1;
+      parents[at + nodes[i].right] = (int64_t)(at + i) * 2;
+    }
+    // Nodes that no split names are not part of the tree.
+    for (size_t i = 0; i < nodes.size(); ++i)
+      if (nodes[i].left < 0 && (i == 0 || parents[at + i] >= 0)) leaves.push_back((uint32_t)(at + i));
+  }
+  const uint32_t elements = mgb_shap_elements(deepest);
+  require(elements != 0, "mgb_predict_contribs: exact contributions need trees of depth at most 16");
+  if (parents.empty()) parents.push_back(-1);
+  DeviceBuffer d_parents, d_leaves;
+  d_parents.upload(parents.data(), parents.size() * sizeof(int64_t));
+  d_leaves.ensure(std::max<size_t>(leaves.size(), 1) * sizeof(uint32_t));
+  d_leaves.upload(leaves.data(), leaves.size() * sizeof(uint32_t));
+  d_root_means_.ensure(std::max<size_t>(roots.size(), 1) * sizeof(float));
+  d_root_means_.upload(roots.data(), roots.size() * sizeof(float));
+  d_shap_table_.ensure(mgb_shap_table_bytes((uint32_t)leaves.size(), elements));
+  kcheck(mgb_shap_paths(d_model_nodes_.as<MgbTreeNode>(), d_parents.as<int64_t>(), d_leaves.as<uint32_t>(),
+                        (uint32_t)leaves.size(), elements, num_feature, d_shap_table_.as<uint32_t>()),
+         "paths");
+  shap_leaves_ = (uint32_t)leaves.size();
+  shap_elements_ = elements;
+  shap_trees_ = end;
+}
+
 std::vector<float> Learner::predict_explain(DMatrix& data, int type, uint32_t end) {
   drain();
   require(type >= 2 && type <= 6, "Prediction type must be 2 to 6 here.");
@@ -1235,6 +1278,28 @@ std::vector<float> Learner::predict_explain(DMatrix& data, int type, uint32_t en
     kcheck(mgb_predict_leaf(X, indptr, indices, data.rows, data.cols, d_model_nodes_.as<MgbTreeNode>(),
                             d_model_offsets_.as<uint32_t>(), end, d_out.as<float>()),
            "leaf prediction");
+  } else if (type == 2 && data.cols < (1u << 24)) {
+    build_paths(end);
+    DeviceBuffer d_base;
+    if (!data.base_margin.empty()) {
+      require(data.base_margin.size() == data.rows, "base_margin must have one value per row.");
+      d_base.upload(data.base_margin.data(), data.rows * sizeof(float));
+    }
+    MgbShap p{};
+    p.X = X;
+    p.indptr = indptr;
+    p.indices = indices;
+    p.table = d_shap_table_.as<uint32_t>();
+    p.root_means = d_root_means_.as<float>();
+    p.base = d_base.get() ? d_base.as<float>() : nullptr;
+    p.out = d_out.as<float>();
+    p.rows = data.rows;
+    p.cols = data.cols;
+    p.leaves = shap_leaves_;
+    p.elements = shap_elements_;
+    p.trees = end;
+    p.base_value = base_margin_value();
+    kcheck(mgb_predict_shap(&p), "contribution prediction");
   } else {
     std::vector<float> means;
     uint32_t deepest = 0;
@@ -1503,6 +1568,7 @@ void Learner::load_model(const Json& input) {
   packed_depth_ = 0;
   packed_fits_ = true;
   packed_uploaded_ = 0;
+  shap_trees_ = SIZE_MAX;
   metrics.clear();  // src/model.cpp:224
   // A loaded model restarts the engine from seed 0 (src/model.cpp:225).
   rng_.seed(0);

@@ -11,7 +11,7 @@
 // there, and every row takes the same number of steps, the deepest tree's
 // depth, with no exit test.
 //
-// Values are compared as order keys (order_key below): NaN's key is the
+// Values are compared as order keys (order_key): NaN's key is the
 // largest word, a split node's word is its threshold's key plus its
 // default_left bit, and a row goes left where its key plus the same bit,
 // modulo 2^32, is below that word.  The bit cancels for every number and
@@ -38,7 +38,6 @@ constexpr uint32_t kStageTrees = 64;           // trees of one staged chunk, at 
 constexpr uint32_t kOffsetWindow = 1024;       // tree offsets held at a time
 constexpr uint32_t kStagePer = 8;              // nodes a thread loads ahead for the next chunk
 constexpr int kWalks = 4;                      // trees a lane walks side by side
-constexpr uint32_t kMissingKey = 0xffffffffu;
 
 struct PredictArgs {
   const float* X;            // dense rows, or a CSR matrix's values
@@ -56,13 +55,6 @@ struct PredictArgs {
   // of a chunk, values of the CSR value buffer.
   uint32_t tile_rows, slices, stride, chunk_trees, value_words, tree_nodes;
 };
-
-// Keys ordered as the numbers are, -0 as +0; every NaN has the largest.
-__device__ __forceinline__ uint32_t order_key(float v) {
-  const uint32_t bits = __float_as_uint(v + 0.0f);
-  const uint32_t key = bits ^ ((uint32_t)((int32_t)bits >> 31) | 0x80000000u);
-  return isnan(v) ? kMissingKey : key;
-}
 
 __device__ __forceinline__ uint32_t node_feature(uint32_t link) { return link >> 17; }
 
