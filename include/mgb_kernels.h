@@ -450,6 +450,13 @@ int mgb_metric_sum(const float* pred, const float* labels, const float* weights,
  * (kernels/radix_sort.metal.h:427-790).  Synchronises. */
 int mgb_metric_auc(const float* pred, const float* labels, const float* weights, uint32_t rows, int pr, double* out,
                    void* workspace, size_t workspace_bytes);
+/* The same without waiting: out is device memory (2 floats / 3 doubles).
+ * mgb_metric_sum_bytes: the scratch mgb_metric_sum needs alone. */
+size_t mgb_metric_sum_bytes(uint32_t rows);
+int mgb_metric_sum_async(const float* pred, const float* labels, const float* weights, uint32_t rows, uint32_t kind,
+                         float parameter, float* out, void* workspace, size_t workspace_bytes);
+int mgb_metric_auc_async(const float* pred, const float* labels, const float* weights, uint32_t rows, int pr,
+                         double* out, void* workspace, size_t workspace_bytes);
 
 #ifdef __cplusplus
 }

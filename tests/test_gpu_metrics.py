@@ -62,6 +62,37 @@ def test_auc_matches_oracle(rows):
                                    O.metric_auc(pred, y, pr=True, weights=weights), rtol=1e-12)
 
 
+@pytest.mark.parametrize("rows,steps", [(2047, 5), (2048, 1), (2049, 2049), (4097, 2), (2_099_201, 3),
+                                        (2_099_201, 1_000_000)])
+def test_auc_steps_across_workgroups(rows, steps):
+    """Steps longer than a workgroup's 2,048 rows, one step in all, and more
+    workgroups than one pass of the prefix takes; exact without weights."""
+    rng = np.random.default_rng(rows + steps)
+    pred = rng.integers(0, steps, size=rows).astype(np.float32)
+    y = (rng.random(rows) < 0.4).astype(np.float32)
+    y[:2] = (1, 0)
+    w = rng.uniform(0.2, 2.0, rows).astype(np.float32)
+    np.testing.assert_array_equal(D.metric_auc(pred, y), O.metric_auc(pred, y))
+    np.testing.assert_allclose(D.metric_auc(pred, y, weights=w), O.metric_auc(pred, y, weights=w), rtol=1e-12)
+    np.testing.assert_allclose(D.metric_auc(pred, y, pr=True, weights=w), O.metric_auc(pred, y, pr=True, weights=w),
+                               rtol=1e-12)
+
+
+def test_eval_of_several_matrices_and_metrics_in_one_line(xgb):
+    """Every matrix's metrics share one copy back: each value is its own."""
+    X, y = W.config1(rows=5000, cols=8)
+    y = (y > 0).astype(np.float32)
+    parts = [(0, 3000), (3000, 3001), (3001, 5000)]
+    mats = [(xgb.DMatrix(X[a:b], label=y[a:b]), f"m{a}") for a, b in parts]
+    names = ["error", "auc", "logloss", "aucpr", "rmse"]
+    bst = xgb.train({"objective": "binary:logistic", "max_depth": 3}, mats[0][0], 3)
+    bst.set_param({"eval_metric": names})
+    line = bst.eval_set(mats, 7)
+    expect = [bst.eval_set([m], 7).split("\t")[1:] for m in mats]
+    assert line == "\t".join(["[7]"] + [v for part in expect for v in part])
+    assert "m3000-auc:nan" in line  # one class only
+
+
 def _expected_line(iteration, evals, metrics):
     """The evaluation line from oracle metric values, printed as the
     reference prints a binary64 with 10 significant digits."""

@@ -1093,19 +1093,23 @@ void Learner::drain() {
   }), "device-to-host copy of the queued rounds");
 }
 
+// Whether every label lies in [0, 1], checked once per label assignment.
+static bool labels_in_unit(DMatrix& d) {
+  if (d.labels_in_unit < 0) {
+    d.labels_in_unit = 1;
+    for (float y : d.labels)
+      if (!(y >= 0 && y <= 1)) { d.labels_in_unit = 0; break; }
+  }
+  return d.labels_in_unit == 1;
+}
+
 void Learner::update(DMatrix& data, int /*iteration*/) {
   configure_check();
   require(data.labels.size() == data.rows, "Labels must be provided for training (one per row).");
   require(data.weights.empty() || data.weights.size() == data.rows, "Number of weights must equal the number of rows.");
   int obj = objective();
   if (obj == 1 || obj == 2) {
-    if (data.labels_in_unit < 0) {
-      // Checked once per label assignment, not every round.
-      data.labels_in_unit = 1;
-      for (float y : data.labels)
-        if (!(y >= 0 && y <= 1)) { data.labels_in_unit = 0; break; }
-    }
-    require(data.labels_in_unit == 1, "label must be in [0,1] for logistic loss.");
+    require(labels_in_unit(data), "label must be in [0,1] for logistic loss.");
   }
   data.quantize((uint32_t)integer("max_bin", 256), bin_layout(), (uint32_t)integer("hip_histogram_features", 0));
   auto t0 = std::chrono::steady_clock::now();
@@ -1341,13 +1345,15 @@ std::string Learner::default_metric() const {
   return (obj == 1 && objective_name() != "reg:logistic") || obj == 2 ? "logloss" : "rmse";
 }
 
-double Learner::metric(DMatrix& d, const float* pred, const std::string& name) {
+std::function<double(const double*)> Learner::metric(DMatrix& d, const float* pred, const std::string& name,
+                                                     double* out) {
   static const std::map<std::string, uint32_t> kinds{
       {"rmse", MGB_METRIC_RMSE}, {"mae", MGB_METRIC_MAE}, {"rmsle", MGB_METRIC_RMSLE},
       {"logloss", MGB_METRIC_LOGLOSS}, {"error", MGB_METRIC_ERROR}, {"mape", MGB_METRIC_MAPE},
       {"mphe", MGB_METRIC_MPHE}, {"poisson-nloglik", MGB_METRIC_POISSON},
       {"gamma-deviance", MGB_METRIC_GAMMA_DEVIANCE}, {"tweedie-nloglik", MGB_METRIC_TWEEDIE},
       {"gamma-nloglik", MGB_METRIC_GAMMA_NLOGLIK}, {"auc", 13}, {"aucpr", 14}};
+  const double nan = std::numeric_limits<double>::quiet_NaN();
   const size_t sep = name.find('@');
   const std::string base = name.substr(0, sep);
   auto it = kinds.find(base);
@@ -1356,16 +1362,22 @@ double Learner::metric(DMatrix& d, const float* pred, const std::string& name) {
   require(d.weights.empty() || d.weights.size() == d.rows, "Evaluation weights must have one entry per row.");
   d.upload_info();
   const float* w = d.weights.empty() ? nullptr : d.d_weights.as<float>();
-  d_metric_ws_.ensure(std::max<size_t>(mgb_metric_workspace_bytes(d.rows), 256));
   if (it->second >= 13) {
-    for (float y : d.labels) require(y >= 0 && y <= 1, "AUC labels must be in [0,1].");
-    if (!d.rows) return std::numeric_limits<double>::quiet_NaN();
-    double out[3];
-    kcheck(mgb_metric_auc(pred, d.d_labels.as<float>(), w, d.rows, it->second == 14, out, d_metric_ws_.get(),
-                          d_metric_ws_.bytes()),
+    require(labels_in_unit(d), "AUC labels must be in [0,1].");
+    if (!d.rows) return [nan](const double*) { return nan; };
+    if (auc_rows_ != d.rows) {
+      auc_bytes_ = mgb_metric_workspace_bytes(d.rows);
+      auc_rows_ = d.rows;
+    }
+    d_metric_ws_.ensure(std::max<size_t>(auc_bytes_, 256));
+    const bool pr = it->second == 14;
+    kcheck(mgb_metric_auc_async(pred, d.d_labels.as<float>(), w, d.rows, pr, out, d_metric_ws_.get(),
+                                d_metric_ws_.bytes()),
            "auc");
-    if (!(out[1] > 0 && out[2] > 0)) return std::numeric_limits<double>::quiet_NaN();
-    return it->second == 13 ? out[0] / (out[1] * out[2]) : out[0];
+    return [pr, nan](const double* v) {
+      if (!(v[1] > 0 && v[2] > 0)) return nan;
+      return pr ? v[0] : v[0] / (v[1] * v[2]);
+    };
   }
   float parameter = 0;
   if (base == "error") parameter = sep == std::string::npos ? 0.5f : std::stof(name.substr(sep + 1));
@@ -1375,27 +1387,46 @@ double Learner::metric(DMatrix& d, const float* pred, const std::string& name) {
     parameter = std::stof(name.substr(sep + 1));
     require(parameter >= 1 && parameter < 2, "Tweedie variance power must be in [1, 2).");
   }
-  float out[2];
-  kcheck(mgb_metric_sum(pred, d.d_labels.as<float>(), w, d.rows, it->second, parameter, out, d_metric_ws_.get(),
-                        d_metric_ws_.bytes()),
+  d_metric_ws_.ensure(mgb_metric_sum_bytes(d.rows));
+  kcheck(mgb_metric_sum_async(pred, d.d_labels.as<float>(), w, d.rows, it->second, parameter,
+                              reinterpret_cast<float*>(out), d_metric_ws_.get(), d_metric_ws_.bytes()),
          "metric");
-  const double mean = out[1] > 0 ? (double)out[0] / (double)out[1] : std::numeric_limits<double>::quiet_NaN();
-  return base == "rmse" || base == "rmsle" ? std::sqrt(mean) : mean;
+  const bool root = base == "rmse" || base == "rmsle";
+  return [root, nan](const double* v) {
+    float sums[2];
+    std::memcpy(sums, v, sizeof(sums));
+    const double mean = sums[1] > 0 ? (double)sums[0] / (double)sums[1] : nan;
+    return root ? std::sqrt(mean) : mean;
+  };
 }
 
+// Every metric of every matrix is queued, and their sums come back in one
+// copy: one wait a round instead of one to three a metric.
 std::string Learner::evaluate(int iteration, const std::vector<DMatrix*>& data, const std::vector<std::string>& names) {
   require(initialized, "Model is not yet initialized (not fitted).");
   if (metrics.empty() && integer("disable_default_eval_metric", 0) == 0) metrics.push_back(default_metric());
-  std::ostringstream os;
-  os << '[' << iteration << ']' << std::setprecision(10);
+  const size_t total = data.size() * metrics.size();
+  d_metric_out_.ensure(std::max<size_t>(total, 1) * 3 * sizeof(double));
+  std::vector<std::function<double(const double*)>> values;
   for (size_t k = 0; k < data.size(); ++k) {
     DMatrix& d = *data[k];
     const float* pred = predict_device(d, false, 0, 0, d_eval_pred_);
     for (auto const& name : metrics) {
       require(d.labels.size() == d.rows, "Evaluation data requires labels.");
-      os << '\t' << names[k] << '-' << name << ':' << metric(d, pred, name);
+      values.push_back(metric(d, pred, name, d_metric_out_.as<double>() + 3 * values.size()));
     }
   }
+  std::vector<double> sums(3 * total);
+  kcheck(download_pinned(d_metric_out_.get(), sums.size() * sizeof(double),
+                         [&](const uint8_t* host) { std::memcpy(sums.data(), host, sums.size() * sizeof(double)); }),
+         "device-to-host copy of the metrics");
+  std::ostringstream os;
+  os << '[' << iteration << ']' << std::setprecision(10);
+  for (size_t k = 0, at = 0; k < data.size(); ++k)
+    for (auto const& name : metrics) {
+      os << '\t' << names[k] << '-' << name << ':' << values[at](sums.data() + 3 * at);
+      ++at;
+    }
   return os.str();
 }
 

@@ -149,9 +149,10 @@ class Learner {
   // "[iteration]\t<name>-<metric>:<value>..." over every metric and matrix
   // (src/learner.cpp:1025-1048).
   std::string evaluate(int iteration, const std::vector<DMatrix*>& data, const std::vector<std::string>& names);
-  // One metric of predictions `pred` (device) against data's labels
-  // (src/metrics.cpp:8-159).
-  double metric(DMatrix& data, const float* pred, const std::string& name);
+  // Queues one metric of predictions `pred` (device) against data's labels
+  // (src/metrics.cpp:8-159), its sums going to `out` (3 doubles' room on the
+  // device); returns the function that gives its value from those sums.
+  std::function<double(const double*)> metric(DMatrix& data, const float* pred, const std::string& name, double* out);
   std::string default_metric() const;
   // eval_metric values in the order first set, each once.
   std::vector<std::string> metrics;
@@ -244,7 +245,9 @@ class Learner {
   std::vector<int32_t> monotone_;         // parsed constraints, cols entries
   std::string monotone_text_ = "()";      // the parameter they were parsed from
   bool monotone_active_ = false;
-  DeviceBuffer d_eval_pred_, d_metric_ws_;
+  DeviceBuffer d_eval_pred_, d_metric_ws_, d_metric_out_;
+  uint32_t auc_rows_ = 0;       // rows whose AUC scratch was sized last,
+  size_t auc_bytes_ = 0;        // and its size
   // Queued rounds: node records (then the node count) at `offset` in d_pending_.
   struct Pending {
     size_t offset, node_bytes;
