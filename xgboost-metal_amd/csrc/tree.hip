@@ -1601,6 +1601,93 @@ __device__ __forceinline__ void score_pair(NodeEval& na, const LaneBins<CH>& la,
   offer_best(nb, mineb, topb, recb, bestb, feature, count, cols);
 }
 
+// A built node's histogram of one feature that the split item builds itself, in
+// LDS: a small matrix's levels without a histogram launch.  The item's W waves
+// add the node's rows (ids and gradient pairs in list order, the feature's codes
+// from its column, which caches hold) and read the bins back; a node whose
+// children will subtract from it has the row written to its bank as well.
+// Bound by launches and the chain of loads: 5,003 x 20, depth 6, a level's
+// 6.1 us histogram and 9.0 us split become one launch (own_level has the
+// sizes).  The codes are gathered, a cache line a row and feature, so that the
+// launch saved pays only while the columns stay in the caches near the CU.
+struct OwnHist {
+  uint32_t g, h;     // LDS byte addresses of bin 0's sums (h: counts with unit Hessians)
+  uint64_t unit_q;   // a row's quantized Hessian with unit Hessians, else 0
+  int64_t* bank;
+  __device__ __forceinline__ void pair(uint32_t bin, bool store, uint64_t& vg, uint64_t& vh) const {
+    vg = *(lds_u64_t*)(uintptr_t)(g + bin * 8);
+    vh = unit_q ? unit_q * *(lds_u32_t*)(uintptr_t)(h + bin * 4) : *(lds_u64_t*)(uintptr_t)(h + bin * 8);
+    if (store) store_pair(bank, bin, vg, vh);
+  }
+};
+
+template <int W>
+__device__ __forceinline__ void item_sync() {
+  if constexpr (W > 1) {
+    __syncthreads();
+  } else {  // one wave: its own LDS operations are in order
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+    __builtin_amdgcn_wave_barrier();
+  }
+}
+
+template <int W, typename BinT>
+__device__ __forceinline__ void own_rows(const Tree& t, const OwnHist& own, const Frontier& node, uint32_t f,
+                                         uint32_t depth, uint32_t first, float sg, float sh) {
+  const uint32_t* rows = t.rows[depth & 1];
+  const float2* gh = t.gh[depth & 1];
+  const BinT* codes = reinterpret_cast<const BinT*>(t.columns) + (uint64_t)f * t.rows_n;
+  constexpr uint32_t kStep = W * kWave;
+  constexpr int kU = 4;  // rows a lane has in flight
+  for (uint32_t i0 = first; i0 < node.count; i0 += kU * kStep) {
+    uint32_t code[kU];
+    float2 v[kU];
+#pragma unroll
+    for (int u = 0; u < kU; ++u) {
+      const uint32_t i = i0 + u * kStep, at = node.begin + (i < node.count ? i : i0);
+      v[u] = gh[at];
+      code[u] = codes[rows[at]];
+    }
+#pragma unroll
+    for (int u = 0; u < kU; ++u) {
+      if (i0 + u * kStep >= node.count) break;
+      const uint32_t bin = min(code[u], t.max_bin);  // the missing code lies above
+      const unsigned long long qg = (unsigned long long)(long long)rintf(v[u].x * sg);
+      if (own.unit_q) {
+        lds_add(own.g + bin * 8, qg);
+        lds_add(own.h + bin * 4, 1u);
+      } else {
+        const unsigned long long qh = (unsigned long long)(long long)rintf(v[u].y * sh);
+        if ((qg | qh) == 0) continue;
+        lds_add(own.g + bin * 8, qg);
+        lds_add(own.h + bin * 8, qh);
+      }
+    }
+  }
+}
+
+template <int W>
+__device__ __forceinline__ OwnHist own_hist(const Tree& t, uint8_t* lds, const Frontier& node, int64_t* bank_row,
+                                            uint32_t f, uint32_t depth, uint32_t first) {
+  const uint32_t B1 = t.bins1;
+  const float sg = t.scales[0], sh = t.scales[1];
+  OwnHist own;
+  own.g = lds_address(lds);
+  own.h = own.g + B1 * 8;
+  own.unit_q = t.unit_hessian ? (uint64_t)(int64_t)rintf(1.0f * sh) : 0;
+  own.bank = bank_row;
+  uint32_t* words = reinterpret_cast<uint32_t*>(lds);
+  for (uint32_t i = first; i < B1 * (t.unit_hessian ? 3u : 4u); i += W * kWave) words[i] = 0;
+  item_sync<W>();
+  if (t.bin_bytes == 1) own_rows<W, uint8_t>(t, own, node, f, depth, first, sg, sh);
+  else own_rows<W, uint16_t>(t, own, node, f, depth, first, sg, sh);
+  item_sync<W>();
+  return own;
+}
+__host__ __device__ inline uint32_t own_hist_bytes(const Tree& t) {
+  return (t.bins1 * (t.unit_hessian ? 12u : 16u) + 15u) / 16u * 16u;
+}
+
 // ---------------------------------------------------------------------------
 // One item = (node pair, feature) below the root, (feature) at the root, and
 // W waves per item with CH consecutive bins per lane, so every bin of the
@@ -1608,10 +1695,13 @@ __device__ __forceinline__ void score_pair(NodeEval& na, const LaneBins<CH>& la,
 // independent items into a 256-thread block with no barrier; for W > 1 a
 // block is one item, so early exits stay block-uniform.  Levels with few
 // items spread each over more waves (CH = 1), wide levels use CH = 4.
+// OWN: the item builds its built node's histogram itself (own_hist; below the
+// root only).
 // ---------------------------------------------------------------------------
-template <int W, int CH>
+template <int W, int CH, bool OWN>
 __global__ __launch_bounds__(W == 1 ? kSplitPack * kWave : W * kWave) void k_split(Tree t, uint32_t depth) {
   constexpr uint32_t kItemsPerBlock = W == 1 ? kSplitPack : 1;  // barriers (W > 1) need whole-block items
+  extern __shared__ __align__(16) uint8_t own_smem[];
   __shared__ uint64_t xtot[kItemsPerBlock][W][4];
   __shared__ float xlo[kItemsPerBlock][2][W];
   __shared__ uint64_t xkey[kItemsPerBlock][2][W];
@@ -1695,12 +1785,22 @@ __global__ __launch_bounds__(W == 1 ? kSplitPack * kWave : W * kWave) void k_spl
   const int64_t* parent = t.hist[(depth - 1) & 1] + ((uint64_t)a.parent_slot * F + f) * B1 * 2;
   int64_t* ob = cur + ((uint64_t)other * F + f) * B1 * 2;
   const bool store_other = depth + 1 < t.max_depth;  // both children are parents at the next level
-  const BuiltHist hb = built_hist(t, cur + ((uint64_t)built * F + f) * B1 * 2, fb, f);
+  int64_t* built_row = cur + ((uint64_t)built * F + f) * B1 * 2;
+  BuiltHist hb;
+  OwnHist own;
+  if constexpr (OWN)
+    own = own_hist<W>(t, own_smem + (size_t)slot_in_block * own_hist_bytes(t), fb, built_row, f, depth,
+                      wave_in_item * kWave + lane);
+  else hb = built_hist(t, built_row, fb, f);
+  auto built_bin = [&](uint32_t bin, bool store, uint64_t& g, uint64_t& v) {
+    if constexpr (OWN) own.pair(bin, store, g, v);
+    else built_pair(hb, bin, store, g, v);
+  };
   const uint32_t count = t.counts[f];
   // Missing slots: they give each child's present-bin totals.
   uint64_t pmg, pmh, xmg = 0, xmh = 0;
   load_pair(parent, MB, pmg, pmh);
-  if (!t.sparse) built_pair(hb, MB, store_other && wave_in_item == 0 && lane == 0, xmg, xmh);
+  if (!t.sparse) built_bin(MB, store_other && wave_in_item == 0 && lane == 0, xmg, xmh);
   LaneBins<CH> x, o;
 #pragma unroll
   for (int j = 0; j < CH; ++j) {
@@ -1708,7 +1808,7 @@ __global__ __launch_bounds__(W == 1 ? kSplitPack * kWave : W * kWave) void k_spl
     if (b0 + j < count) {
       uint64_t pg, ph;
       load_pair(parent, b0 + j, pg, ph);
-      built_pair(hb, b0 + j, store_other, xg, xh);
+      built_bin(b0 + j, store_other, xg, xh);
       og = pg - xg;
       oh = ph - xh;
       if (store_other) store_pair(ob, b0 + j, og, oh);
@@ -1727,7 +1827,7 @@ __global__ __launch_bounds__(W == 1 ? kSplitPack * kWave : W * kWave) void k_spl
     // values: its present parent bins minus the built child's).
     xmg = (uint64_t)fb.sum_g - all[0];
     xmh = (uint64_t)fb.sum_h - all[1];
-    if (store_other && wave_in_item == 0 && lane == 0) store_pair(hb.bank, MB, xmg, xmh);
+    if (store_other && wave_in_item == 0 && lane == 0) store_pair(built_row, MB, xmg, xmh);
   }
   const uint64_t omg = pmg - xmg, omh = pmh - xmh;
   if (store_other && wave_in_item == 0 && lane == 0) store_pair(ob, MB, omg, omh);
@@ -2719,6 +2819,7 @@ uint32_t split_waves(uint32_t max_bin) {
 // Items of a level (upper bound known on the host) below about eight waves
 // per CU take one bin per lane on four times the waves: shallow levels are
 // latency bound, deep ones throughput bound.
+template <bool OWN>
 int launch_split(const Tree& t, uint32_t depth, uint32_t items) {
   const uint32_t w4 = split_waves(t.max_bin);
   if (w4 * kWave * 4 < t.max_bin) { set_error("max_bin too large for the split kernel"); return -1; }
@@ -2731,23 +2832,49 @@ int launch_split(const Tree& t, uint32_t depth, uint32_t items) {
   const bool spread = (w4 >= 4 ? (uint64_t)items < 2048 : (uint64_t)items * w4 < 2048) && w4 * 4 <= 16;
   const uint32_t w = spread ? 4 * w4 : w4;
   const dim3 grid(w == 1 ? div_up(items, kSplitPack) : items), block(w == 1 ? kSplitPack * kWave : w * kWave);
+  const uint32_t lds = OWN ? own_hist_bytes(t) * (w == 1 ? kSplitPack : 1) : 0;
+#define MGB_SPLIT_CASE(W, CH)                                                                            \
+  {                                                                                                      \
+    auto fn = k_split<W, CH, OWN>;                                                                       \
+    if (lds > 48 * 1024 && check(hipFuncSetAttribute((const void*)fn,                                    \
+                                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds), \
+                                 "hipFuncSetAttribute(split LDS)"))                                      \
+      return -1;                                                                                         \
+    launch(MGB_PROF_SPLIT, fn, grid, block, lds, t, depth);                                              \
+    break;                                                                                               \
+  }
   if (!spread) {
     switch (w) {
-      case 1: launch(MGB_PROF_SPLIT, k_split<1, 4>, grid, block, 0, t, depth); break;
-      case 2: launch(MGB_PROF_SPLIT, k_split<2, 4>, grid, block, 0, t, depth); break;
-      case 4: launch(MGB_PROF_SPLIT, k_split<4, 4>, grid, block, 0, t, depth); break;
-      case 8: launch(MGB_PROF_SPLIT, k_split<8, 4>, grid, block, 0, t, depth); break;
-      default: launch(MGB_PROF_SPLIT, k_split<16, 4>, grid, block, 0, t, depth); break;
+      case 1: MGB_SPLIT_CASE(1, 4)
+      case 2: MGB_SPLIT_CASE(2, 4)
+      case 4: MGB_SPLIT_CASE(4, 4)
+      case 8: MGB_SPLIT_CASE(8, 4)
+      default: MGB_SPLIT_CASE(16, 4)
     }
   } else {
     switch (w) {
-      case 4: launch(MGB_PROF_SPLIT, k_split<4, 1>, grid, block, 0, t, depth); break;
-      case 8: launch(MGB_PROF_SPLIT, k_split<8, 1>, grid, block, 0, t, depth); break;
-      default: launch(MGB_PROF_SPLIT, k_split<16, 1>, grid, block, 0, t, depth); break;
+      case 4: MGB_SPLIT_CASE(4, 1)
+      case 8: MGB_SPLIT_CASE(8, 1)
+      default: MGB_SPLIT_CASE(16, 1)
     }
   }
+#undef MGB_SPLIT_CASE
   MGB_LAUNCH_CHECK("k_split");
   return 0;
+}
+
+// Whether a level's split items build their own histograms: below the root, on
+// matrices of at most kOwnRows rows, where its nodes hold at most kOwnNode
+// rows on average (an item walks a node's rows alone), unless the caller asks
+// for deeper histograms from the columns.  50 rounds, histogram launches
+// against own histograms: 5,003 x 20 depth 6 7.9 -> 6.5 ms, 16,000 x 64 depth 8
+// (logistic) 15.1 -> 12.5, 32,000 x 32 depth 6 8.0 -> 7.2, 60,000 x 64 depth 8
+// 14.2 -> 13.4, 60,000 x 32 depth 6 8.5 -> 8.3 (every level: 8.4); beyond, the
+// gathered codes cost more than the launch: 100,000 x 32 depth 6 8.8 -> 9.1,
+// 262,144 x 64 16.6 -> 20.4.
+constexpr uint32_t kOwnRows = 65536, kOwnNode = 16384;
+bool own_level(const Tree& t, uint32_t depth) {
+  return depth > 0 && t.columns && t.column_levels <= 1 && t.rows_n <= kOwnRows && (t.rows_n >> depth) <= kOwnNode;
 }
 
 // Select + partition of a level: `grid` partition workgroups plus the
@@ -2952,11 +3079,15 @@ int mgb_grow_tree(const MgbTreeShape* shape, const MgbMatrix* m, const void* bin
     }
     const uint32_t hgrid = hist_grid_for(t, level_hist_tasks(t, depth));
     const uint32_t pgrid = level_part_grid(t, depth);
-    if ((m->bin_bytes == 1 ? dispatch_hist<uint8_t>(t, depth, hgrid) : dispatch_hist<uint16_t>(t, depth, hgrid)))
-      return -1;
     uint32_t max_nodes = 1u << depth;
     uint32_t items = depth == 0 ? shape->cols : (max_nodes / 2) * shape->cols;
-    if (launch_split(t, depth, items)) return -1;
+    if (own_level(t, depth)) {
+      if (launch_split<true>(t, depth, items)) return -1;
+    } else {
+      if ((m->bin_bytes == 1 ? dispatch_hist<uint8_t>(t, depth, hgrid) : dispatch_hist<uint16_t>(t, depth, hgrid)))
+        return -1;
+      if (launch_split<false>(t, depth, items)) return -1;
+    }
     if ((m->bin_bytes == 1 ? launch_apply<uint8_t>(t, depth, pgrid) : launch_apply<uint16_t>(t, depth, pgrid)))
       return -1;
   }
@@ -3119,7 +3250,7 @@ int mgb_grow_tree_csr(const MgbTreeShape* shape, const MgbCsrMatrix* m, const ui
     if (csr_histogram(t, m->bin_bytes, depth, root_columns, hgrid, zx)) return -1;
     uint32_t max_nodes = 1u << depth;
     uint32_t items = depth == 0 ? shape->cols : (max_nodes / 2) * shape->cols;
-    if (launch_split(t, depth, items)) return -1;
+    if (launch_split<false>(t, depth, items)) return -1;
     const uint32_t pgrid = level_part_grid(t, depth);
     if ((m->bin_bytes == 1 ? launch_apply<uint8_t>(t, depth, pgrid) : launch_apply<uint16_t>(t, depth, pgrid)))
       return -1;
