@@ -124,3 +124,32 @@ def test_partition_modes_train_identical_models(xgb):
     csr = sps.csr_matrix((values, indices, indptr), shape=(20000, 300))
     _same_with_both_partitions(xgb, xgb.DMatrix(csr, label=yc),
                                {"max_depth": 6, "max_bin": 64, "objective": "binary:logistic", "eta": 0.1}, 4)
+
+
+@pytest.mark.parametrize("rows,cols,share,depth,max_bin", [
+    (1, 3, 0.5, 2, 16), (64, 2, 1.0, 3, 16), (1023, 7, 0.5, 5, 256), (1024, 40, 0.05, 6, 64), (1025, 300, 0.02, 6, 256),
+    (5000, 4, 0.9, 9, 1024), (20000, 200, 0.05, 8, 256), (70000, 5, 0.01, 4, 256)])
+def test_csr_stable_partition_trains_like_claims(xgb, rows, cols, share, depth, max_bin):
+    """The stable partition of a CSR matrix takes a tile's directions from a
+    stretch of the split feature's column (or, where a tile's rows lie far
+    apart, from a search in each row); tiles that claim their ranges search
+    each row.  Both train the same trees, with stored NaN, empty rows and
+    columns, u8 and u16 codes."""
+    import scipy.sparse as sp
+    rng = np.random.default_rng(rows + cols)
+    dense = rng.normal(size=(rows, cols)).astype(np.float32)
+    keep = rng.random(dense.shape) < share
+    keep[:, cols // 2] &= cols < 4  # an empty column
+    r, c = np.nonzero(keep)
+    values = dense[r, c]
+    values[rng.random(len(values)) < 0.03] = np.nan
+    csr = sp.csr_matrix((values, (r, c)), shape=dense.shape)
+    y = (np.where(keep, dense, 0).sum(axis=1) + 0.3 * rng.normal(size=rows)).astype(np.float32)
+    models = []
+    for stable in (0, 1):
+        d = xgb.DMatrix(csr, label=y)
+        bst = xgb.train({"max_depth": depth, "max_bin": max_bin, "eta": 0.4, "hip_stable_partition": stable}, d, 4)
+        trees = json.loads(bst.save_raw("json"))["learner"]["gradient_booster"]["model"]["trees"]
+        models.append((trees, bst.predict(d, output_margin=True)))
+    assert models[0][0] == models[1][0]
+    np.testing.assert_array_equal(models[0][1], models[1][1])
