@@ -1738,6 +1738,93 @@ __host__ __device__ inline uint32_t own_hist_bytes(const Tree& t) {
   return (t.bins1 * (t.unit_hessian ? 12u : 16u) + 15u) / 16u * 16u;
 }
 
+// One wave's bins that hold anything, closed up: inclusive prefix sums and the
+// bins they belong to.  A bin without mass has the sums of a neighbour whose
+// order is smaller -- forward the bin before it, backward the one after -- so
+// neither of its candidates can be the first strictly greater one (at either
+// end of the feature one side is empty and the candidate invalid).
+constexpr uint32_t kClosedBins = 4 * kWave;
+struct ClosedBins {
+  uint64_t g[kClosedBins], h[kClosedBins];
+  uint16_t bin[kClosedBins];
+};
+
+// In kernels that close bins up, none in the others.
+struct NoBins {};
+template <bool CLOSED>
+struct ClosedStore { using type = NoBins; };
+template <>
+struct ClosedStore<true> { using type = ClosedBins; };
+
+// score_node for an item of one wave and four bins a lane, over the bins with
+// mass only: a sparse feature's built node fills few of its 256 bins (1M x 2,000,
+// 20 entries a row), and the bounds of 64 candidates a direction cost the wave
+// the same vector operations as one.  94.9 -> 89.1 us a launch at that matrix's
+// wide levels; dense matrices fill their bins and keep score_node.
+__device__ __forceinline__ void score_closed(NodeEval& n, const LaneBins<4>& lb, uint64_t pre_g, uint64_t pre_h,
+                                             uint32_t b0, uint32_t count, int eg, int eh, float mcw, bool filter,
+                                             float lambda, const MgbSplitParams& p, ClosedBins& c, SplitRec* rec,
+                                             unsigned long long* node_best, uint32_t feature, uint32_t cols) {
+  const uint32_t lane = lane_id();
+  uint32_t rank = 0, total = 0, here = 0;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const bool mass = lb.g[j] != (j ? lb.g[j - 1] : 0) || lb.h[j] != (j ? lb.h[j - 1] : 0);
+    const uint64_t m = __ballot(mass);  // bins past the feature's last hold nothing
+    here |= mass ? 1u << j : 0u;
+    rank = __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, rank));
+    total += (uint32_t)__popcll(m);
+  }
+  __builtin_amdgcn_wave_barrier();
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    if ((here >> j) & 1u) {
+      c.g[rank] = pre_g + lb.g[j];
+      c.h[rank] = pre_h + lb.h[j];
+      c.bin[rank] = (uint16_t)(b0 + j);
+      ++rank;
+    }
+  }
+  item_sync<1>();
+  float hi_f[4], hi_b[4], lo = -INFINITY;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    hi_f[r] = hi_b[r] = -INFINITY;
+    if ((uint32_t)r * kWave >= total) continue;  // uniform
+    const uint32_t e = r * kWave + lane;
+    if (e < total) {
+      float l;
+      gain_bounds(n, c.g[e], c.h[e], eg, eh, mcw, filter, lambda, l, hi_f[r]);
+      lo = fmaxf(lo, l);
+      if (n.has_missing) {
+        const uint64_t xg = e ? c.g[e - 1] : 0, xh = e ? c.h[e - 1] : 0;
+        gain_bounds(n, n.tg - (n.pg - xg), n.th - (n.ph - xh), eg, eh, mcw, filter, lambda, l, hi_b[r]);
+        lo = fmaxf(lo, l);
+      }
+    }
+  }
+  const float node_lo = wave_max_f32(lo);
+  uint32_t mask = 0;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    if (hi_f[r] > -INFINITY && hi_f[r] >= node_lo) mask |= 1u << (2 * r);
+    if (hi_b[r] > -INFINITY && hi_b[r] >= node_lo) mask |= 2u << (2 * r);
+  }
+  while (mask) {
+    const uint32_t k = (uint32_t)__builtin_ctz(mask);
+    mask &= mask - 1;
+    const uint32_t e = (k >> 1) * kWave + lane, b = c.bin[e];
+    const bool backward = (k & 1) != 0;
+    const uint32_t at = backward ? e - 1 : e;  // e = 0 backward: nothing lies before
+    const uint64_t ig = backward && e == 0 ? 0 : c.g[at], ih = backward && e == 0 ? 0 : c.h[at];
+    const uint64_t lg = backward ? n.tg - (n.pg - ig) : ig;
+    const uint64_t lh = backward ? n.th - (n.ph - ih) : ih;
+    try_candidate(n, lg, lh, backward ? 2 * count - 1 - b : b, eg, eh, mcw, p);
+  }
+  const uint64_t mine = candidate_key(n);
+  offer_best(n, mine, wave_max_u64(mine), rec, node_best, feature, count, cols);
+}
+
 // ---------------------------------------------------------------------------
 // One item = (node pair, feature) below the root, (feature) at the root, and
 // W waves per item with CH consecutive bins per lane, so every bin of the
@@ -1746,12 +1833,15 @@ __host__ __device__ inline uint32_t own_hist_bytes(const Tree& t) {
 // block is one item, so early exits stay block-uniform.  Levels with few
 // items spread each over more waves (CH = 1), wide levels use CH = 4.
 // OWN: the item builds its built node's histogram itself (own_hist; below the
-// root only).
+// root only).  CLOSED (one wave, four bins a lane): bins without mass are left
+// out of the scoring (score_closed).
 // ---------------------------------------------------------------------------
-template <int W, int CH, bool OWN>
+template <int W, int CH, bool OWN, bool CLOSED>
 __global__ __launch_bounds__(W == 1 ? kSplitPack * kWave : W * kWave) void k_split(Tree t, uint32_t depth) {
   constexpr uint32_t kItemsPerBlock = W == 1 ? kSplitPack : 1;  // barriers (W > 1) need whole-block items
   extern __shared__ __align__(16) uint8_t own_smem[];
+  static_assert(!CLOSED || (W == 1 && CH == 4), "closed bins: one wave, four bins a lane");
+  __shared__ typename ClosedStore<CLOSED>::type closed[kItemsPerBlock];
   __shared__ typename StripeStore<CH>::type s_cells[kItemsPerBlock * W];
   __shared__ uint64_t xtot[kItemsPerBlock][W][4];
   __shared__ float xlo[kItemsPerBlock][2][W];
@@ -1887,7 +1977,12 @@ __global__ __launch_bounds__(W == 1 ? kSplitPack * kWave : W * kWave) void k_spl
   const int32_t mono = t.monotone ? t.monotone[f] : 0;
   node_begin(ex, (uint64_t)fb.sum_g, (uint64_t)fb.sum_h, xmg, xmh, eg, eh, t.sp, fb.lower, fb.upper, mono);
   node_begin(eo, (uint64_t)fo.sum_g, (uint64_t)fo.sum_h, omg, omh, eg, eh, t.sp, fo.lower, fo.upper, mono);
-  if constexpr (W > 1 && CH > 1) {
+  if constexpr (CLOSED) {
+    score_closed(ex, x, pre[0], pre[1], b0, count, eg, eh, mcw, filter, lambda, t.sp, closed[slot_in_block],
+                 t.recs + (uint64_t)built * F + f, best_bank(t, depth) + built * kKeyWays, f, t.cols);
+    score_closed(eo, o, pre[2], pre[3], b0, count, eg, eh, mcw, filter, lambda, t.sp, closed[slot_in_block],
+                 t.recs + (uint64_t)other * F + f, best_bank(t, depth) + other * kKeyWays, f, t.cols);
+  } else if constexpr (W > 1 && CH > 1) {
     // Several waves and bins per lane: both children share each exchange's
     // barrier (C4's wide levels: split 1.374 -> 1.352 ms per round).  With
     // one wave per item there is no barrier to share (scored together
@@ -2979,9 +3074,9 @@ int launch_split(const Tree& t, uint32_t depth, uint32_t items) {
   const uint32_t w = spread ? 4 * w4 : w4;
   const dim3 grid(w == 1 ? div_up(items, kSplitPack) : items), block(w == 1 ? kSplitPack * kWave : w * kWave);
   const uint32_t lds = OWN ? own_hist_bytes(t) * (w == 1 ? kSplitPack : 1) : 0;
-#define MGB_SPLIT_CASE(W, CH)                                                                            \
+#define MGB_SPLIT_CASE(W, CH, CLOSED)                                                                    \
   {                                                                                                      \
-    auto fn = k_split<W, CH, OWN>;                                                                       \
+    auto fn = k_split<W, CH, OWN, CLOSED>;                                                                       \
     if (lds > 48 * 1024 && check(hipFuncSetAttribute((const void*)fn,                                    \
                                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds), \
                                  "hipFuncSetAttribute(split LDS)"))                                      \
@@ -2991,18 +3086,19 @@ int launch_split(const Tree& t, uint32_t depth, uint32_t items) {
   if (!spread) {
     switch (w) {
       case 1:
-        MGB_SPLIT_CASE(1, 4)
+        if (t.sparse) MGB_SPLIT_CASE(1, 4, true)
+        else MGB_SPLIT_CASE(1, 4, false)
         break;
-      case 2: MGB_SPLIT_CASE(2, 4) break;
-      case 4: MGB_SPLIT_CASE(4, 4) break;
-      case 8: MGB_SPLIT_CASE(8, 4) break;
-      default: MGB_SPLIT_CASE(16, 4) break;
+      case 2: MGB_SPLIT_CASE(2, 4, false) break;
+      case 4: MGB_SPLIT_CASE(4, 4, false) break;
+      case 8: MGB_SPLIT_CASE(8, 4, false) break;
+      default: MGB_SPLIT_CASE(16, 4, false) break;
     }
   } else {
     switch (w) {
-      case 4: MGB_SPLIT_CASE(4, 1) break;
-      case 8: MGB_SPLIT_CASE(8, 1) break;
-      default: MGB_SPLIT_CASE(16, 1) break;
+      case 4: MGB_SPLIT_CASE(4, 1, false) break;
+      case 8: MGB_SPLIT_CASE(8, 1, false) break;
+      default: MGB_SPLIT_CASE(16, 1, false) break;
     }
   }
 #undef MGB_SPLIT_CASE
