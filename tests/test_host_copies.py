@@ -1,0 +1,50 @@
+"""Dense matrices keep the values they were given, around the sizes where the
+host copy takes large pages (4 MiB) and several threads (8 MiB on, up to eight
+shares of 4 MiB, the last one ragged)."""
+import numpy as np
+import pytest
+
+import device_lib as D
+
+
+@pytest.mark.parametrize("rows,cols", [
+    (1, 1), (1, (1 << 20) - 1), (1 << 20, 1), ((1 << 20) + 1, 1), ((1 << 21) - 1, 1), (1 << 21, 1), (700001, 3),
+    (131071, 73)])
+@pytest.mark.parametrize("form", ["float32", "strided", "float64", "missing"])
+def test_dense_values_survive(xgb, rows, cols, form):
+    n = rows * cols
+    values = np.arange(n, dtype=np.float32).reshape(rows, cols)  # below 2^24: all distinct
+    given, missing = values, np.nan
+    if form == "strided":
+        wide = np.full((rows, cols + 1), np.nan, np.float32)
+        wide[:, :cols] = values
+        given = wide[:, :cols]
+    elif form == "float64":
+        given = values.astype(np.float64)
+    elif form == "missing":
+        missing = float(n - 1)
+    got = xgb.DMatrix(given, missing=missing).get_data()
+    want = values.reshape(-1)[:-1] if form == "missing" else values.reshape(-1)
+    assert got.shape == values.shape
+    np.testing.assert_array_equal(got.data, want)
+    np.testing.assert_array_equal(got.indices, np.tile(np.arange(cols), rows)[:len(want)])
+
+
+def test_empty_matrix(xgb):
+    assert xgb.DMatrix(np.empty((0, 4), np.float32)).num_row() == 0
+
+
+# Uploads from 8 MiB on go through pinned chunks of 2 MiB, filled by six threads
+# with two chunks each: below, at and past the limit, ragged last chunks, and
+# several turns of every chunk.
+@pytest.mark.gpu
+@pytest.mark.parametrize("nbytes", [
+    (8 << 20) - 1, 8 << 20, (8 << 20) + 1, (12 << 20) + 4097, (24 << 20) + 2, (26 << 20) - 3, (70 << 20) + 5])
+def test_large_uploads(nbytes):
+    rng = np.random.default_rng(nbytes)
+    for _ in range(2):
+        host = rng.integers(0, 256, nbytes, dtype=np.uint8)
+        dev = D.Device.of(host)
+        host_after = host.copy()
+        host[:] = 0  # the copy is complete when the call returns
+        np.testing.assert_array_equal(dev.read(np.uint8, nbytes), host_after)

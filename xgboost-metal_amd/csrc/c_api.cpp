@@ -150,10 +150,10 @@ float load_value(const ArrayView& v, int64_t offset) {
   throw Error("Unsupported array dtype.");
 }
 
-std::vector<float> to_vector(const ArrayView& v) {
+HostFloats to_vector(const ArrayView& v) {
   int64_t n = 1;
   for (auto d : v.shape) n *= d;
-  std::vector<float> out((size_t)n);
+  HostFloats out((size_t)n);
   // C-contiguous float32: one copy.
   bool contiguous = v.kind == 'f' && v.itemsize == 4;
   for (size_t k = 0, step = 4; contiguous && k < v.shape.size(); ++k) {
@@ -162,7 +162,7 @@ std::vector<float> to_vector(const ArrayView& v) {
     step *= (size_t)v.shape[axis];
   }
   if (contiguous) {
-    if (n) std::memcpy(out.data(), v.data, (size_t)n * sizeof(float));
+    copy_large(out.data(), v.data, (size_t)n * sizeof(float));
     return out;
   }
   if (v.shape.size() == 1) {
@@ -186,7 +186,7 @@ float config_missing(const char* config) {
   return (float)m.number();
 }
 
-void apply_missing(std::vector<float>& data, float missing) {
+void apply_missing(HostFloats& data, float missing) {
   if (std::isnan(missing)) return;
   for (auto& x : data) if (x == missing) x = NAN;
 }
@@ -236,7 +236,7 @@ std::shared_ptr<DMatrix> columnar_matrix(const char* text, float missing) {
   require(columns.is_array() && columns.size() > 0, "Columnar data must be a non-empty list of array interfaces.");
   auto d = std::make_shared<DMatrix>();
   d->cols = (uint32_t)columns.size();
-  std::vector<std::vector<float>> cols;
+  std::vector<HostFloats> cols;
   for (auto const& c : columns.items()) {
     std::string one = c.dump();
     ArrayView v = parse_interface(one.c_str());
@@ -708,7 +708,8 @@ int XGDMatrixCreateFromMat(const float* data, bst_ulong nrow, bst_ulong ncol, fl
   auto d = std::make_shared<DMatrix>();
   d->rows = (uint32_t)nrow;
   d->cols = (uint32_t)ncol;
-  d->data.assign(data, data + nrow * ncol);
+  d->data.resize((size_t)nrow * ncol);
+  copy_large(d->data.data(), data, d->data.size() * sizeof(float));
   apply_missing(d->data, missing);
   *out = new_handle(std::move(d));
   API_END
@@ -734,7 +735,7 @@ int XGDMatrixFree(DMatrixHandle handle) {
 int XGDMatrixSetInfoFromInterface(DMatrixHandle handle, char const* field, char const* data) {
   API_BEGIN
   ArrayView v = parse_interface(data);
-  std::vector<float> values = to_vector(v);
+  const HostFloats values = to_vector(v);
   matrix(handle)->set_info(field, values.data(), values.size());
   API_END
 }

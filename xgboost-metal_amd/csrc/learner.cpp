@@ -65,7 +65,9 @@ void DMatrix::upload() {
 
 uint64_t DMatrix::nonmissing() const {
   uint64_t n = 0;
-  for (float x : sparse ? values : data) n += !std::isnan(x);
+  const float* x = sparse ? values.data() : data.data();
+  const size_t stored = sparse ? values.size() : data.size();
+  for (size_t i = 0; i < stored; ++i) n += !std::isnan(x[i]);
   return n;
 }
 

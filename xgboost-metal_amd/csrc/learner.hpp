@@ -16,6 +16,7 @@
 #include <string>
 #include <vector>
 
+#include "host_memory.hpp"
 #include "json.hpp"
 #include "mgb_kernels.h"
 
@@ -57,7 +58,7 @@ int download_pinned(const void* src, size_t bytes, const std::function<void(cons
 struct DMatrix {
   uint64_t id = 0;                    // unique per matrix; keys the prediction cache
   uint32_t rows = 0, cols = 0;
-  std::vector<float> data;            // row-major, NaN marks missing (dense matrices)
+  HostFloats data;                    // row-major, NaN marks missing (dense matrices)
   // CSR matrices (sparse = true): rows+1 offsets, strictly increasing column
   // indices within a row, values (NaN marks missing; absent entries too).
   bool sparse = false;
