@@ -24,7 +24,20 @@ namespace {
 // ---------------------------------------------------------------------------
 constexpr uint32_t kQuantThreads = 1024;
 constexpr uint32_t kQuantCutsLds = 68 * 1024;   // bytes of staged cuts per workgroup (64 features of 256 cuts, 16 of 1024)
-constexpr uint32_t kQuantChunkCodes = 8192;     // codes per chunk (LDS tile)
+constexpr uint32_t kQuantPer = 8;               // codes a thread per chunk
+constexpr uint32_t kQuantChunkCodes = kQuantPer * kQuantThreads;  // codes per chunk (LDS tile)
+// Workgroups of a launch: two a CU, as the staged cuts allow.  Each stages its
+// cuts once, twice the words of a chunk's codes.
+constexpr uint32_t kQuantGroups = 512;
+
+// Sets *flag where any thread of the workgroup has `found`.  One store a
+// workgroup, and none where the flag is seen set: an atomic from each wave took
+// its turn on the word (100,000 x 32, 15% missing: 16,384 of them, 190 us).
+__device__ __forceinline__ void raise_flag(uint32_t* flag, bool found) {
+  if (__syncthreads_or(found) && threadIdx.x == 0 &&
+      __hip_atomic_load(flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0)
+    __hip_atomic_store(flag, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
 
 // Address of code (r, f) of a bin matrix.
 template <typename BinT>
@@ -33,34 +46,64 @@ __device__ __forceinline__ BinT* code_at(BinT* bins, const MgbMatrix& m, uint64_
   return reinterpret_cast<BinT*>(reinterpret_cast<uint8_t*>(bins) + (uint64_t)g * m.group_stride + r * m.row_stride) + j;
 }
 
-// tile_features and chunk_rows are powers of two; the cuts of feature j sit
-// at s_cuts + j * (cut_stride + 1) (an odd stride, so that the searches of
-// different features start in different LDS banks).  columns (may be NULL)
-// receives the same codes column-major: code (r, f) at columns[f * rows + r].
+// tile_features and chunk_rows are powers of two, a chunk is kQuantPer codes a
+// thread; the cuts of feature j sit at s_cuts + j * (cut_stride + 1) (an odd
+// stride, so that the searches of different features start in different LDS
+// banks), NaN past the last.  columns (may be NULL) receives the same codes
+// column-major: code (r, f) at columns[f * rows + r].
+//
+// Bound by the searches' LDS reads and the stores: a thread's eight values are
+// loaded together and searched in step, no branch among them, and codes leave
+// in 4-byte words of kUnit where the layout's rows and the matrix allow
+// (words, column_words).  Against a value and a branching search at a time and
+// stores of single codes: 262,144 x 64, 256 cuts, 130 -> 56 us (2,048 workgroups
+// that each stage the cuts: 117), 1.5M x 128, 1,024 cuts, 1,537 -> 825.
 template <typename BinT>
-__global__ __launch_bounds__(kQuantThreads) void k_quantize(const float* __restrict__ X, const float* __restrict__ cuts,
+__global__ __launch_bounds__(kQuantThreads, 8) void k_quantize(const float* __restrict__ X, const float* __restrict__ cuts,
                                                             const uint32_t* __restrict__ counts, MgbMatrix m,
                                                             uint32_t tile_shift, uint32_t chunk_shift, uint32_t chunks,
+                                                            uint32_t pitch, bool words, bool column_words,
                                                             BinT* __restrict__ bins, BinT* __restrict__ columns,
                                                             uint32_t* __restrict__ any_missing) {
+  constexpr uint32_t kUnit = 4 / sizeof(BinT);  // codes of a word
   extern __shared__ __align__(16) uint8_t q_smem[];
   const uint32_t tile_features = 1u << tile_shift, chunk_rows = 1u << chunk_shift;
   const uint32_t stride = m.cut_stride + 1;
   float* s_cuts = reinterpret_cast<float*>(q_smem);  // tile_features x stride
   uint32_t* s_count = reinterpret_cast<uint32_t*>(s_cuts + (uint64_t)tile_features * stride);
-  BinT* s_codes = reinterpret_cast<BinT*>(s_count + tile_features);  // chunk_rows x tile_features
+  BinT* s_codes = reinterpret_cast<BinT*>(s_count + tile_features);  // chunk_rows x pitch
   const uint32_t G = m.group_features;
   const uint32_t padded = (m.cols + G - 1) / G * G;
   const uint32_t f0 = blockIdx.y << tile_shift;
   const uint32_t nf = padded - f0 < tile_features ? padded - f0 : tile_features;
   for (uint32_t j = threadIdx.x; j < tile_features; j += blockDim.x) s_count[j] = f0 + j < m.cols ? counts[f0 + j] : 0u;
-  for (uint32_t j = 0; j < nf; ++j) {
-    if (f0 + j >= m.cols) break;
-    const float* src = cuts + (uint64_t)(f0 + j) * m.cut_stride;
-    for (uint32_t c = threadIdx.x; c < m.cut_stride; c += blockDim.x) s_cuts[j * stride + c] = src[c];
+  {
+    const uint32_t here = f0 < m.cols ? min(nf, m.cols - f0) : 0u;
+    uint32_t j = threadIdx.x / stride, c = threadIdx.x % stride;
+    const uint32_t dj = kQuantThreads / stride, dc = kQuantThreads % stride;
+#pragma unroll 4
+    for (uint32_t i = threadIdx.x; i < here * stride; i += kQuantThreads) {
+      const bool cut = c < m.cut_stride && c < counts[f0 + j];
+      s_cuts[i] = cut ? cuts[(uint64_t)(f0 + j) * m.cut_stride + c] : __uint_as_float(0x7fc00000u);
+      j += dj;
+      c += dc;
+      if (c >= stride) {
+        c -= stride;
+        ++j;
+      }
+    }
   }
   __syncthreads();
+  // The search's first step: the largest power of two that is at most cut_stride.
+  const uint32_t top = 1u << (31 - __builtin_clz(m.cut_stride | 1u));
   bool missing = false;
+  // This thread's feature of the tile, its first row of a chunk and the step
+  // (kQuantThreads is a multiple of tile_features, kQuantPer steps fill a chunk).
+  const uint32_t j0 = threadIdx.x & (tile_features - 1), first_row = threadIdx.x >> tile_shift;
+  const uint32_t row_step = kQuantThreads >> tile_shift;
+  const bool there = f0 + j0 < m.cols;
+  const float* column = s_cuts + (there ? j0 : 0u) * stride;
+  const uint32_t count0 = s_count[j0];
   const uint64_t row0 = (uint64_t)blockIdx.x * chunks << chunk_shift;
   const uint32_t codes = chunk_rows << tile_shift;
   for (uint32_t chunk = 0; chunk < chunks; ++chunk) {
@@ -68,52 +111,83 @@ __global__ __launch_bounds__(kQuantThreads) void k_quantize(const float* __restr
     if (r0 >= m.rows) break;
     const uint32_t nr = m.rows - r0 < chunk_rows ? (uint32_t)(m.rows - r0) : chunk_rows;
     // Rows in order, features fastest: consecutive threads read a row's
-    // consecutive values.
-    for (uint32_t i = threadIdx.x; i < codes; i += blockDim.x) {
-      const uint32_t rr = i >> tile_shift, j = i & (tile_features - 1);
-      if (rr >= nr || j >= nf) continue;
-      const uint32_t f = f0 + j;
-      BinT code = (BinT)m.missing_code;
-      if (f < m.cols) {
-        const float v = X[(r0 + rr) * m.cols + f];
-        const uint32_t count = s_count[j];
-        if (!isnan(v) && count) {
-          const float* column = s_cuts + j * stride;
-          uint32_t lo = 0, hi = count;
-          while (lo < hi) {
-            const uint32_t mid = lo + (hi - lo) / 2;
-            if (v >= column[mid]) lo = mid + 1;
-            else hi = mid;
-          }
-          code = (BinT)(lo < count - 1 ? lo : count - 1);
-        } else {
-          missing = true;
-        }
+    // consecutive values, and a thread's are of one feature.
+    float v[kQuantPer];
+    uint32_t lo[kQuantPer];
+#pragma unroll
+    for (uint32_t u = 0; u < kQuantPer; ++u) {
+      const uint32_t rr = first_row + u * row_step;
+      v[u] = there && rr < nr ? X[(r0 + rr) * m.cols + f0 + j0] : 0.0f;
+      lo[u] = 0;
+    }
+    for (uint32_t bit = top; bit; bit >>= 1) {
+#pragma unroll
+      for (uint32_t u = 0; u < kQuantPer; ++u) {
+        // lo + bit cuts lie at or below v if the last of them does.
+        const float cut = column[min(lo[u] + bit - 1, m.cut_stride)];
+        lo[u] += v[u] >= cut ? bit : 0u;
       }
-      s_codes[i] = code;
+    }
+    if (j0 < nf) {
+#pragma unroll
+      for (uint32_t u = 0; u < kQuantPer; ++u) {
+        const uint32_t rr = first_row + u * row_step;
+        if (rr >= nr) break;
+        BinT code = (BinT)m.missing_code;
+        if (there) {
+          if (!isnan(v[u]) && count0) code = (BinT)min(lo[u], count0 - 1);
+          else missing = true;
+        }
+        s_codes[rr * pitch + j0] = code;
+      }
     }
     __syncthreads();
+    auto put_columns = [&](BinT* out, uint32_t features) {  // consecutive threads along a column
+      if (column_words) {
+        const uint32_t units = chunk_rows / kUnit, unit_shift = 31 - __builtin_clz(units);
+        for (uint32_t i = threadIdx.x; i < units << tile_shift; i += blockDim.x) {
+          const uint32_t rr = (i & (units - 1)) * kUnit, j = i >> unit_shift;
+          if (rr >= nr || j >= features) continue;
+          uint32_t word = 0;
+#pragma unroll
+          for (uint32_t k = 0; k < kUnit; ++k) word |= (uint32_t)s_codes[(rr + k) * pitch + j] << (8 * sizeof(BinT) * k);
+          *reinterpret_cast<uint32_t*>(out + (uint64_t)(f0 + j) * m.rows + r0 + rr) = word;
+        }
+      } else {
+        for (uint32_t i = threadIdx.x; i < codes; i += blockDim.x) {
+          const uint32_t rr = i & (chunk_rows - 1), j = i >> chunk_shift;
+          if (rr < nr && j < features) out[(uint64_t)(f0 + j) * m.rows + r0 + rr] = s_codes[rr * pitch + j];
+        }
+      }
+    };
     if (m.row_stride == sizeof(BinT) && G == 1) {
-      // A column-major matrix: consecutive threads along a column.
-      for (uint32_t i = threadIdx.x; i < codes; i += blockDim.x) {
-        const uint32_t rr = i & (chunk_rows - 1), j = i >> chunk_shift;
-        if (rr < nr && j < nf) *code_at(bins, m, r0 + rr, f0 + j) = s_codes[(rr << tile_shift) + j];
+      put_columns(bins, nf);  // a column-major matrix
+    } else if (words) {
+      // Words in the layout's own order: along a row (row-major), or down a
+      // group's rows (group-major).
+      const uint32_t per_group = G / kUnit, tile_units = tile_features / kUnit;
+      const bool by_group = m.row_stride == (uint64_t)G * sizeof(BinT) && per_group <= tile_units;
+      const uint32_t inner = by_group ? per_group : tile_units, inner_shift = 31 - __builtin_clz(inner);
+      const uint32_t group_shift = 31 - __builtin_clz(G);
+      for (uint32_t i = threadIdx.x; i < codes / kUnit; i += blockDim.x) {
+        const uint32_t w = i & (inner - 1), rest = i >> inner_shift;
+        const uint32_t rr = rest & (chunk_rows - 1), j = (w + (rest >> chunk_shift) * inner) * kUnit;
+        if (rr >= nr || j >= nf) continue;
+        const uint32_t f = f0 + j, g = f >> group_shift;
+        const uint32_t word = *reinterpret_cast<const uint32_t*>(s_codes + rr * pitch + j);
+        *reinterpret_cast<uint32_t*>(reinterpret_cast<uint8_t*>(bins) + (uint64_t)g * m.group_stride +
+                                     (r0 + rr) * m.row_stride + (f & (G - 1)) * sizeof(BinT)) = word;
       }
     } else {
       for (uint32_t i = threadIdx.x; i < codes; i += blockDim.x) {
         const uint32_t rr = i >> tile_shift, j = i & (tile_features - 1);
-        if (rr < nr && j < nf) *code_at(bins, m, r0 + rr, f0 + j) = s_codes[i];
+        if (rr < nr && j < nf) *code_at(bins, m, r0 + rr, f0 + j) = s_codes[rr * pitch + j];
       }
     }
-    if (columns) {
-      for (uint32_t i = threadIdx.x; i < codes; i += blockDim.x) {
-        const uint32_t rr = i & (chunk_rows - 1), j = i >> chunk_shift;
-        if (rr < nr && j < nf && f0 + j < m.cols) columns[(uint64_t)(f0 + j) * m.rows + r0 + rr] = s_codes[(rr << tile_shift) + j];
-      }
-    }
+    if (columns) put_columns(columns, f0 < m.cols ? min(nf, m.cols - f0) : 0u);
     __syncthreads();
   }
-  if (__any(missing) && lane_id() == 0) atomicOr(any_missing, 1u);
+  raise_flag(any_missing, missing);
 }
 
 // ---------------------------------------------------------------------------
@@ -453,11 +527,22 @@ __global__ __launch_bounds__(kBaseThreads) void k_base_score(const float* __rest
   }
 }
 
-__global__ void k_any_missing(const float* __restrict__ data, uint64_t count, uint32_t* __restrict__ flag) {
+// Bound by the read; a wave stops at its first NaN.
+constexpr uint32_t kScanThreads = 256, kScanBlocks = 1024;
+__global__ __launch_bounds__(kScanThreads) void k_any_missing(const float* __restrict__ data, uint64_t count,
+                                                              uint32_t* __restrict__ flag) {
+  constexpr uint32_t kBatch = 8;  // values a thread has in flight
+  const uint64_t threads = (uint64_t)gridDim.x * kScanThreads;
   bool missing = false;
-  for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < count; i += (uint64_t)gridDim.x * blockDim.x)
-    missing |= isnan(data[i]);
-  if (__any(missing) && lane_id() == 0) atomicOr(flag, 1u);
+  for (uint64_t i0 = (uint64_t)blockIdx.x * kScanThreads + threadIdx.x; i0 < count && !missing; i0 += kBatch * threads) {
+    float v[kBatch];
+#pragma unroll
+    for (uint32_t u = 0; u < kBatch; ++u) v[u] = data[i0 + u * threads < count ? i0 + u * threads : i0];
+#pragma unroll
+    for (uint32_t u = 0; u < kBatch; ++u) missing |= isnan(v[u]);
+    missing = __any(missing);
+  }
+  raise_flag(flag, missing);
 }
 
 // Prediction transform of binary:logistic (sigmoid of the margin, the same
@@ -536,8 +621,8 @@ static int quantize(const float* X, const float* cuts, const uint32_t* counts, c
     return -1;
   }
   // Features per workgroup: the largest power of two (at most 64) whose cuts
-  // fit the staging budget; rows in chunks of kQuantChunkCodes codes, and as
-  // many chunks per workgroup as keep about 2048 workgroups busy.
+  // fit the staging budget; rows in chunks of kQuantChunkCodes codes, spread
+  // evenly over at most about kQuantGroups workgroups.
   const uint32_t padded = (uint32_t)(groups * G);
   uint32_t tile_shift = 6;
   while (tile_shift > 0 && ((((uint64_t)1 << tile_shift) * (m->cut_stride + 1) * 4 > kQuantCutsLds) ||
@@ -547,22 +632,30 @@ static int quantize(const float* X, const float* cuts, const uint32_t* counts, c
   while ((1u << (chunk_shift + 1 + tile_shift)) <= kQuantChunkCodes) ++chunk_shift;
   const uint32_t tiles = (padded + (1u << tile_shift) - 1) >> tile_shift;
   const uint64_t row_chunks = (m->rows + (1ull << chunk_shift) - 1) >> chunk_shift;
-  const uint32_t chunks =
-      (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(8, row_chunks * tiles / 2048));
+  const uint32_t chunks = (uint32_t)((row_chunks * tiles + kQuantGroups - 1) / kQuantGroups);
   const dim3 grid((uint32_t)((row_chunks + chunks - 1) / chunks), tiles);
-  const uint32_t lds = (1u << tile_shift) * ((m->cut_stride + 1) * 4 + 4) + (1u << (chunk_shift + tile_shift)) * m->bin_bytes;
+  // Words of codes where a group and a tile hold whole ones and the rows start
+  // aligned; columns likewise.  Wide tiles pad their rows by a word: a column's
+  // codes then lie in different banks.
+  const uint32_t unit = 4 / m->bin_bytes;
+  const uint32_t pitch = (1u << tile_shift) + (tile_shift >= 4 ? unit : 0u);
+  const bool words = G >= unit && (1u << tile_shift) >= unit && (uintptr_t)bins % 4 == 0;
+  const bool column_matrix = G == 1 && m->row_stride == m->bin_bytes;
+  const bool column_words = m->rows % unit == 0 && (1u << chunk_shift) >= unit && (uintptr_t)columns % 4 == 0 &&
+                            (!column_matrix || (uintptr_t)bins % 4 == 0);
+  const uint32_t lds = (1u << tile_shift) * ((m->cut_stride + 1) * 4 + 4) + ((pitch * m->bin_bytes) << chunk_shift);
   if (m->bin_bytes == 1) {
     if (check(hipFuncSetAttribute((const void*)k_quantize<uint8_t>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds),
               "hipFuncSetAttribute(k_quantize)"))
       return -1;
     hipLaunchKernelGGL(k_quantize<uint8_t>, grid, dim3(kQuantThreads), lds, stream(), X, cuts, counts, *m, tile_shift,
-                       chunk_shift, chunks, (uint8_t*)bins, (uint8_t*)columns, any_missing);
+                       chunk_shift, chunks, pitch, words, column_words, (uint8_t*)bins, (uint8_t*)columns, any_missing);
   } else {
     if (check(hipFuncSetAttribute((const void*)k_quantize<uint16_t>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds),
               "hipFuncSetAttribute(k_quantize)"))
       return -1;
     hipLaunchKernelGGL(k_quantize<uint16_t>, grid, dim3(kQuantThreads), lds, stream(), X, cuts, counts, *m, tile_shift,
-                       chunk_shift, chunks, (uint16_t*)bins, (uint16_t*)columns, any_missing);
+                       chunk_shift, chunks, pitch, words, column_words, (uint16_t*)bins, (uint16_t*)columns, any_missing);
   }
   MGB_LAUNCH_CHECK("k_quantize");
   return 0;
@@ -638,7 +731,7 @@ int mgb_fill_f32(float* data, uint64_t count, float value) {
 
 int mgb_any_missing(const float* data, uint64_t count, uint32_t* flag) {
   if (!count) return 0;
-  hipLaunchKernelGGL(k_any_missing, dim3(grid_for(count, 256, 4096)), dim3(256), 0, stream(), data, count, flag);
+  hipLaunchKernelGGL(k_any_missing, dim3(grid_for(count, kScanThreads, kScanBlocks)), dim3(kScanThreads), 0, stream(), data, count, flag);
   MGB_LAUNCH_CHECK("k_any_missing");
   return 0;
 }
