@@ -344,16 +344,18 @@ int mgb_predict(const float* X, uint32_t rows, uint32_t cols, const MgbTreeNode*
 
 /* A tree packed for prediction.  link: bits 0-15 the distance in nodes from a
  * split node to its left child (the right child follows the left one; 0: a
- * leaf), bit 16 default_left, bits 17-31 the feature.  word: a leaf's value
- * (binary32), or a split node's threshold as an order key -- the sign bit of a
- * number not below 0 flipped, every bit of a negative one, -0 as +0 -- plus
- * default_left.  A leaf's feature is the model's feature count and its
- * default_left 1, so that a walk stays there.  Trees follow one another: tree
- * t is nodes [offsets[t], offsets[t + 1]), children after their parents, both
- * offsets even (an unused node may fill the end). */
+ * leaf), bit 16 default_left, bits 17-31 the feature.  word: the bits of a
+ * leaf's value (binary32) exclusive-or MGB_PACKED_LEAF, or a split node's
+ * threshold as an order key -- the sign bit of a number not below 0 flipped,
+ * every bit of a negative one, -0 as +0 -- plus default_left.  A leaf's feature
+ * is the model's feature count, its default_left 1 and its word not 0, so that
+ * a walk stays there.  Trees follow one another: tree t is nodes [offsets[t],
+ * offsets[t + 1]), children after their parents, both offsets even (an unused
+ * leaf may fill the end). */
 typedef struct {
   uint32_t word, link;
 } MgbPackedNode;
+#define MGB_PACKED_LEAF 0x7f800001u  /* a signalling NaN, which no packed leaf is */
 #define MGB_PACKED_FEATURES 32768u  /* packed models have fewer features */
 #define MGB_PACKED_DISTANCE 65535u  /* largest distance to a left child */
 /* Margins (or, for objective 1 = logistic, their sigmoid) of the trees of

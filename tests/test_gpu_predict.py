@@ -158,3 +158,103 @@ def test_logistic_output_is_the_sigmoid_of_the_margin(xgb, rows):
     # Rounding of e^x, two sums and a division: a few units of 2^-24.
     np.testing.assert_allclose(bst.predict(xgb.DMatrix(X)), 1.0 / (1.0 + np.exp(-margin.astype(np.float64))),
                                rtol=4e-7, atol=0)
+
+
+def _special_values(rng, forest, X):
+    """Leaves of +0 and -0 at every depth (the leaves nearest the root among
+    them) and thresholds at zeros, infinities and the rows' own values."""
+    special = [0.0, -0.0, np.inf, -np.inf]
+    flat = X[~np.isnan(X)]
+    for t in forest:
+        for k, left in enumerate(t["left_children"]):
+            u = rng.random()
+            if left < 0:
+                t["split_conditions"][k] = 0.0 if u < 0.5 else -0.0 if u < 0.6 else t["split_conditions"][k]
+            elif u < 0.5:
+                t["split_conditions"][k] = float(special[rng.integers(4)] if u < 0.2 or not len(flat) else rng.choice(flat))
+    X[rng.random(X.shape) < 0.1] = 0.0
+    X[rng.random(X.shape) < 0.1] = -0.0
+    X[rng.random(X.shape) < 0.05] = np.inf
+    X[rng.random(X.shape) < 0.05] = -np.inf
+
+
+def _stump(value):
+    return {"left_children": [-1], "right_children": [-1], "split_indices": [0], "split_conditions": [value],
+            "default_left": [0], "parents": [2147483647], "loss_changes": [0], "sum_hessian": [0], "base_weights": [0]}
+
+
+def _same_bits(got, expect):
+    np.testing.assert_array_equal(np.asarray(got, np.float32).view(np.uint32), expect.view(np.uint32))
+
+
+@pytest.mark.parametrize("rows,cols,trees,depth,shuffle", [
+    (1, 1, 1, 1, False), (16, 9, 130, 5, True), (300, 6, 3, 12, False), (12287, 31, 20, 6, True),
+    (12289, 31, 20, 6, False), (20000, 64, 70, 8, False), (13000, 6, 2, 13, False), (12300, 1200, 5, 5, False)])
+def test_leaves_of_zero_hold_the_walk(xgb, rows, cols, trees, depth, shuffle):
+    """Single leaves of +0 before, between and after deeper trees, +0 and -0
+    leaves above the deepest level, thresholds equal to the values compared."""
+    rng = np.random.default_rng(rows * 7 + cols)
+    forest = [_random_tree(rng, cols, depth if t % 3 == 0 else int(rng.integers(1, depth + 1)), shuffle)
+              for t in range(trees)]
+    X = _values(rng, rows, cols, 0.1)
+    _special_values(rng, forest, X)
+    forest = [_stump(0.0), *forest[:1], _stump(0.0), *forest[1:], _stump(-0.0), _stump(0.0)]
+    bst = _booster(xgb, forest, cols)
+    loaded = json.loads(bst.save_raw("json"))["learner"]["gradient_booster"]["model"]["trees"]
+    expect = _margins(loaded, X, 0.25)
+    _same_bits(bst.predict(xgb.DMatrix(X)), expect)
+    _same_bits(bst.inplace_predict(X), expect)
+    base = rng.normal(size=rows).astype(np.float32)
+    base[::2] = -0.0
+    _same_bits(bst.predict(xgb.DMatrix(X, base_margin=base)), _margins(loaded, X, base))
+    _same_bits(bst.predict(xgb.DMatrix(X), iteration_range=(0, 1)), _margins(loaded[:1], X, 0.25))
+    _same_bits(bst.predict(xgb.DMatrix(X), iteration_range=(2, len(loaded))), _margins(loaded[2:], X, 0.25))
+    _same_bits(_booster(xgb, [_stump(0.0)], cols).predict(xgb.DMatrix(X)), np.full(rows, 0.25, np.float32))
+
+
+@pytest.mark.parametrize("rows,cols,trees,depth", [(5, 40, 9, 4), (6145, 33, 70, 6), (13000, 2000, 20, 7)])
+def test_leaves_of_zero_hold_the_walk_csr(xgb, rows, cols, trees, depth):
+    import scipy.sparse as sp
+    rng = np.random.default_rng(rows + cols)
+    used = np.sort(rng.choice(cols, size=min(cols, 50), replace=False))
+    forest = [_random_tree(rng, len(used), 1 + t % depth, False) for t in range(trees)]
+    small = _values(rng, rows, len(used), 0.6)
+    _special_values(rng, forest, small)
+    forest = [_stump(0.0), *forest, _stump(0.0)]
+    r, c = np.nonzero(~np.isnan(small))
+    csr = sp.csr_matrix((small[r, c], (r, used[c])), shape=(rows, cols))
+    wide = [dict(t, split_indices=[int(used[f]) for f in t["split_indices"]]) for t in forest]
+    bst = _booster(xgb, wide, cols)
+    loaded = json.loads(bst.save_raw("json"))["learner"]["gradient_booster"]["model"]["trees"]
+    plain = [dict(t, split_conditions=l["split_conditions"]) for t, l in zip(forest, loaded)]
+    expect = _margins(plain, small, 0.25)
+    _same_bits(bst.predict(xgb.DMatrix(csr)), expect)
+    _same_bits(bst.inplace_predict(csr), expect)
+
+
+@pytest.mark.parametrize("rows", [700, 13000])
+def test_fits_with_leaves_of_zero(xgb, rows):
+    """A learning rate that reaches 0, rows without weight and gradients of 0
+    leave +0 and -0 leaves; a new matrix of the training rows gets the training
+    margins."""
+    rng = np.random.default_rng(rows)
+    X = _values(rng, rows, 6, 0.1)
+    y = (np.nan_to_num(X[:, 0]) * np.nan_to_num(X[:, 1])).astype(np.float32)
+    weight = (np.nan_to_num(X[:, 2]) > 0).astype(np.float32)
+    params = {"max_depth": 5, "max_bin": 32, "eta": 0.4, "min_child_weight": 0, "lambda": 0}
+    schedule = xgb.callback.LearningRateScheduler(lambda r: 0.4 if r < 3 else 0.0)
+
+    def nothing(margin, dtrain):
+        return np.zeros(rows, np.float32), np.ones(rows, np.float32)
+
+    fits = [xgb.train(params, xgb.DMatrix(X, label=y), 6, callbacks=[schedule]),
+            xgb.train(params, xgb.DMatrix(X, label=y, weight=weight), 4),
+            xgb.train(params, xgb.DMatrix(X, label=y), 3, obj=nothing)]
+    for bst in fits:
+        trees = json.loads(bst.save_raw("json"))["learner"]["gradient_booster"]["model"]["trees"]
+        base = float(json.loads(bst.save_raw("json"))["learner"]["learner_model_param"]["base_score"].strip("[]"))
+        expect = _margins(trees, X, base)
+        np.testing.assert_array_equal(bst.predict(xgb.DMatrix(X), output_margin=True), expect)
+        np.testing.assert_array_equal(bst.inplace_predict(X), expect)
+    zeros = json.loads(fits[0].save_raw("json"))["learner"]["gradient_booster"]["model"]["trees"][-1]
+    assert any(l < 0 and v == 0 for l, v in zip(zeros["left_children"], zeros["split_conditions"]))

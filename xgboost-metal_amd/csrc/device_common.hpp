@@ -121,14 +121,6 @@ __device__ __forceinline__ uint32_t block_exclusive_u32(uint32_t v, uint32_t* sh
   return result;
 }
 
-// Keys ordered as the numbers are, -0 as +0; every NaN has the largest.
-constexpr uint32_t kMissingKey = 0xffffffffu;
-__device__ __forceinline__ uint32_t order_key(float v) {
-  const uint32_t bits = __float_as_uint(v + 0.0f);
-  const uint32_t key = bits ^ ((uint32_t)((int32_t)bits >> 31) | 0x80000000u);
-  return isnan(v) ? kMissingKey : key;
-}
-
 // Exact binary32 <-> integer helpers.
 __device__ __forceinline__ float bits_to_float(uint32_t b) { return __uint_as_float(b); }
 

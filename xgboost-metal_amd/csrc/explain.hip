@@ -15,6 +15,7 @@
 #include <cmath>
 
 #include "device_common.hpp"
+#include "packed_tree.hpp"
 
 namespace mgb {
 namespace {

@@ -8,6 +8,8 @@
 #include <limits>
 #include <sstream>
 
+#include "packed_tree.hpp"
+
 namespace mgb {
 
 void require(bool ok, const std::string& message) {
@@ -508,47 +510,6 @@ void Learner::upload_model() {
   uploaded_trees_ = trees.size();
   model_version_ = trees.size();
 }
-
-namespace {
-
-// Appends a tree in packed form, breadth first (a trained tree's own order);
-// false if it does not fit: a feature or a distance out of range, a NaN
-// threshold, or nodes that are not a tree.
-bool pack_tree(const std::vector<MgbTreeNode>& t, uint32_t features, std::vector<MgbPackedNode>& out,
-               uint32_t& deepest) {
-  std::vector<std::pair<uint32_t, uint32_t>> order;  // (node id, depth) by packed position
-  order.reserve(t.size());
-  if (t.empty()) return false;
-  order.emplace_back(0u, 0u);
-  for (size_t i = 0; i < order.size(); ++i) {
-    const auto [id, depth] = order[i];
-    const MgbTreeNode& n = t[id];
-    MgbPackedNode packed;
-    if (n.left < 0) {
-      std::memcpy(&packed.word, &n.leaf, sizeof(float));
-      packed.link = (features << 17) | (1u << 16);
-    } else {
-      const size_t distance = order.size() - i;
-      if (n.feature < 0 || (uint32_t)n.feature >= features || std::isnan(n.threshold) || distance > MGB_PACKED_DISTANCE ||
-          (size_t)n.left >= t.size() || n.right < 0 || (size_t)n.right >= t.size() || order.size() + 2 > t.size())
-        return false;
-      const float threshold = n.threshold + 0.0f;
-      uint32_t bits;
-      std::memcpy(&bits, &threshold, sizeof(bits));
-      const uint32_t go = n.default_left ? 1u : 0u;
-      packed.word = (bits & 0x80000000u ? ~bits : bits | 0x80000000u) + go;
-      packed.link = (uint32_t)distance | (go << 16) | ((uint32_t)n.feature << 17);
-      order.emplace_back((uint32_t)n.left, depth + 1);
-      order.emplace_back((uint32_t)n.right, depth + 1);
-      deepest = std::max(deepest, depth + 1);
-    }
-    out.push_back(packed);
-  }
-  if (out.size() % 2) out.push_back(MgbPackedNode{0, (features << 17) | (1u << 16)});  // trees start at even nodes
-  return true;
-}
-
-}  // namespace
 
 bool Learner::pack_model() {
   if (num_feature >= MGB_PACKED_FEATURES) return false;

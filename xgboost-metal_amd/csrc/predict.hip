@@ -3,13 +3,13 @@
 // entries follow default_left, and a row's margin adds one leaf a tree in tree
 // order, in binary32.
 //
-// A packed node is 8 bytes: a word to compare (a leaf's value) and a link --
-// the distance to the left child (16 bits; the right child follows the left),
-// default_left (1 bit) and the feature (15 bits).  A leaf's distance is 0, its
-// feature is one past the model's features -- no row has it, so it reads as
-// missing -- and its default is left: a walk that has reached a leaf stays
-// there, and every row takes the same number of steps, the deepest tree's
-// depth, with no exit test.
+// A packed node is 8 bytes: a word to compare (a leaf's value, coded so that
+// it is not 0) and a link -- the distance to the left child (16 bits; the right
+// child follows the left), default_left (1 bit) and the feature (15 bits).  A
+// leaf's distance is 0, its feature is one past the model's features -- no row
+// has it, so it reads as missing -- and its default is left, where 0 is below
+// its word: a walk that has reached a leaf stays there, and every row takes the
+// same number of steps, the deepest tree's depth, with no exit test.
 //
 // Values are compared as order keys (order_key): NaN's key is the
 // largest word, a split node's word is its threshold's key plus its
@@ -23,6 +23,7 @@
 
 #include "binary32_exp.hpp"
 #include "device_common.hpp"
+#include "packed_tree.hpp"
 
 namespace mgb {
 namespace {
@@ -55,13 +56,6 @@ struct PredictArgs {
   // of a chunk, values of the CSR value buffer.
   uint32_t tile_rows, slices, stride, chunk_trees, value_words, tree_nodes;
 };
-
-__device__ __forceinline__ uint32_t node_feature(uint32_t link) { return link >> 17; }
-
-// Distance from a node to the child that a row with this key goes to.
-__device__ __forceinline__ uint32_t step_of(uint32_t word, uint32_t link, uint32_t key) {
-  return (link & 0xffffu) + (key + ((link >> 16) & 1u) < word ? 0u : 1u);
-}
 
 __device__ __forceinline__ float finish(const PredictArgs& a, float sum) {
   return a.transform ? sigmoid_binary32(sum) : sum;
@@ -119,18 +113,18 @@ __device__ __forceinline__ void walk(const Nodes& nodes, uint32_t (&at)[kWalks],
 #pragma unroll
     for (int j = 0; j < N; ++j) {
       asm volatile("" : "+v"(link[j]));
-      key[j] = row(node_feature(link[j]));
+      key[j] = row(packed_feature(link[j]));
     }
 #pragma unroll
     for (int j = 0; j < N; ++j) {
       asm volatile("" : "+v"(key[j]));
-      at[j] += step_of(word[j], link[j], key[j]);
+      at[j] += packed_step(word[j], link[j], key[j]);
       link[j] = nodes.link(at[j]);
       word[j] = nodes.word(at[j]);
     }
   }
 #pragma unroll
-  for (int j = 0; j < N; ++j) leaf[j] = __uint_as_float(word[j]);
+  for (int j = 0; j < N; ++j) leaf[j] = packed_leaf(word[j]);
 }
 
 template <typename Row>
@@ -390,7 +384,7 @@ __global__ __launch_bounds__(kDirectWaves * kWave) void k_predict_direct(Predict
       for (uint32_t d = 0; d < a.depth; ++d) {
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
-          at[j] += step_of(n[j].x, n[j].y, key_of(node_feature(n[j].y)));
+          at[j] += packed_step(n[j].x, n[j].y, key_of(packed_feature(n[j].y)));
           n[j] = a.nodes[at[j]];
         }
       }
@@ -398,7 +392,7 @@ __global__ __launch_bounds__(kDirectWaves * kWave) void k_predict_direct(Predict
       for (int j = 0; j < 2; ++j) {
         const uint32_t base = t0 + j * kWave;
         const uint32_t m = base < a.trees ? min(a.trees - base, (uint32_t)kWave) : 0u;
-        for (uint32_t q = 0; q < m; ++q) sum = sum + __uint_as_float(__builtin_amdgcn_readlane(n[j].x, q));
+        for (uint32_t q = 0; q < m; ++q) sum = sum + packed_leaf(__builtin_amdgcn_readlane(n[j].x, q));
       }
     }
     if (lane == 0) a.out[r] = finish(a, sum);
