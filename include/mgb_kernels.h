@@ -408,25 +408,32 @@ int mgb_predict_contribs(const float* X, const uint64_t* indptr, const uint32_t*
  * depth (0: deeper than 16), mgb_shap_table_bytes the table's size.
  * mgb_shap_paths fills it for `count` leaves: leaves[k] the leaf's place in
  * `nodes`, parents[i] the place of node i's parent times two, plus one where
- * node i is its left child (-1 for a root).  mgb_predict_shap: out as
+ * node i is its left child (-1 for a root).  used: the `features` features that
+ * the trees split on, rising (device memory), which the table and the scratch
+ * then number; NULL: every feature of the matrix.  mgb_predict_shap: out as
  * mgb_predict_contribs' (rows x (cols + 1), the bias last: base[r], or
- * base_value if base is NULL, plus root_means[0 .. trees)), rows dense or CSR;
- * allocates its scratch (at most 256 MB, or one 64-row tile's). */
+ * base_value if base is NULL, plus root_means[0 .. trees)), rows dense or CSR,
+ * used and features as the table's.  Allocates mgb_shap_scratch_bytes (host
+ * arithmetic alone: rows, leaves and features are read), at most 256 MB; 0: so
+ * many features, or rows of so many, that mgb_predict_contribs is the better
+ * way, and mgb_predict_shap fails. */
 typedef struct {
   const float* X;
   const uint64_t* indptr;
   const uint32_t* indices;
   const uint32_t* table;
+  const uint32_t* used;
   const float* root_means;
   const float* base;
   float* out;
-  uint32_t rows, cols, leaves, elements, trees;
+  uint32_t rows, cols, leaves, elements, trees, features;
   float base_value;
 } MgbShap;
 uint32_t mgb_shap_elements(uint32_t depth);
 size_t mgb_shap_table_bytes(uint32_t leaves, uint32_t elements);
+size_t mgb_shap_scratch_bytes(const MgbShap* p);
 int mgb_shap_paths(const MgbTreeNode* nodes, const int64_t* parents, const uint32_t* leaves, uint32_t count,
-                   uint32_t elements, uint32_t cols, uint32_t* table);
+                   uint32_t elements, const uint32_t* used, uint32_t features, uint32_t* table);
 int mgb_predict_shap(const MgbShap* p);
 
 /* ---- evaluation metrics (src/metrics.cpp:8-159) ------------------------- */

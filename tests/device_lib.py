@@ -24,6 +24,18 @@ class MgbTreeShape(ctypes.Structure):
                 ("compact_sampled", ctypes.c_uint32), ("stable_partition", ctypes.c_uint32)]
 
 
+class MgbShap(ctypes.Structure):
+    _fields_ = [(name, ctypes.c_void_p) for name in ("X", "indptr", "indices", "table", "used", "root_means", "base",
+                                                     "out")] + \
+               [(name, ctypes.c_uint32) for name in ("rows", "cols", "leaves", "elements", "trees", "features")] + \
+               [("base_value", ctypes.c_float)]
+
+
+# MgbTreeNode
+TREE_NODE = np.dtype([("left", np.int32), ("right", np.int32), ("parent", np.int32), ("feature", np.int32),
+                      ("threshold", np.float32), ("leaf", np.float32), ("cover", np.float32), ("gain", np.float32),
+                      ("default_left", np.uint32), ("base_weight", np.float32)])
+
 _lib = None
 
 

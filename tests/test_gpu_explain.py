@@ -366,3 +366,109 @@ def test_contributions_over_path_lengths_and_widths(xgb, rows, cols, depth, roun
         np.testing.assert_allclose(part.sum(axis=1), bst.predict(d, output_margin=True, iteration_range=(0, 1)),
                                    rtol=0, atol=2e-5 * scale)
         np.testing.assert_array_equal(bst.predict(d, pred_contribs=True), exact.astype(np.float32))
+
+
+def _covered_forest(xgb, rng, cols, trees, depth, features=None):
+    """Boosted-looking trees with covers, split features among `features`
+    (default: all), loaded as a model; and the trees."""
+    features = np.arange(cols) if features is None else features
+    out = []
+    for _ in range(trees):
+        t = {key: [] for key in ("left_children", "right_children", "split_indices", "split_conditions", "default_left",
+                                 "parents", "sum_hessian")}
+
+        def add(parent, cover):
+            for key, v in (("left_children", -1), ("right_children", -1), ("split_indices", 0),
+                           ("split_conditions", float(np.float32(rng.normal() * 0.1))), ("default_left", 0),
+                           ("parents", parent), ("sum_hessian", float(cover))):
+                t[key].append(v)
+            return len(t["left_children"]) - 1
+
+        level = {add(2147483647, 4096): 0}
+        k = 0
+        while k < len(t["left_children"]):
+            cover = t["sum_hessian"][k]
+            if level[k] < depth and cover >= 2 and (level[k] == 0 or rng.random() < 0.97):
+                a = int(rng.integers(1, cover))
+                t["split_indices"][k] = int(rng.choice(features))
+                t["split_conditions"][k] = float(np.float32(rng.normal()))
+                t["default_left"][k] = int(rng.integers(2))
+                t["left_children"][k] = add(k, a)
+                t["right_children"][k] = add(k, cover - a)
+                level[t["left_children"][k]] = level[t["right_children"][k]] = level[k] + 1
+            k += 1
+        t["loss_changes"] = t["base_weights"] = [0] * len(t["left_children"])
+        out.append(t)
+    model = {"version": [3, 5, 0], "learner": {
+        "attributes": {}, "feature_names": [], "feature_types": [],
+        "learner_model_param": {"base_score": "0.25", "num_class": "0", "num_feature": str(cols), "num_target": "1"},
+        "objective": {"name": "reg:squarederror"},
+        "gradient_booster": {"name": "gbtree", "model": {"trees": out, "tree_info": [0] * trees}}}}
+    return xgb.Booster(model_file=bytearray(json.dumps(model).encode())), out
+
+
+@pytest.mark.parametrize("rows,cols,trees,depth,some", [
+    (1, 65, 9, 5, False), (130, 65, 2, 2, False), (65, 290, 30, 4, False), (1, 2000, 60, 8, False),
+    (130, 2000, 12, 6, False), (3, 100_000, 40, 7, False), (200, 40_000, 3, 3, True), (64, 5000, 20, 6, True)])
+def test_contributions_of_wide_rows(xgb, rows, cols, trees, depth, some):
+    """Tables over the features that some split names, more rows than a tile,
+    columns that no split names (their contributions are 0); exact values of a
+    few rows in binary64, and the sums of all against the margins."""
+    import scipy.sparse as sp
+    rng = np.random.default_rng(rows + cols)
+    features = np.sort(rng.choice(cols, size=25, replace=False)) if some else None
+    if some:
+        features[-1] = cols - 1
+    bst, forest = _covered_forest(xgb, rng, cols, trees, depth, features)
+    used = sorted({f for t in forest for f, l in zip(t["split_indices"], t["left_children"]) if l >= 0})
+    X = np.full((rows, cols), np.nan, np.float32)
+    keep = rng.random((rows, len(used))) < 0.6
+    X[:, used] = np.where(keep, rng.normal(size=keep.shape).astype(np.float32), np.nan)
+    extra = rng.integers(0, cols, size=rows)
+    X[np.arange(rows), extra] = 1.0
+    d = xgb.DMatrix(X) if cols <= 5000 else None
+    r, c = np.nonzero(~np.isnan(X))
+    csr = xgb.DMatrix(sp.csr_matrix((X[r, c], (r, c)), shape=X.shape))
+    got = bst.predict(csr, pred_contribs=True)
+    if d is not None:
+        np.testing.assert_array_equal(bst.predict(d, pred_contribs=True), got)
+    margin = bst.predict(csr, output_margin=True).astype(np.float64)
+    scale = max(1.0, np.abs(margin).max())
+    np.testing.assert_allclose(got.astype(np.float64).sum(axis=1), margin, rtol=0, atol=2e-5 * scale)
+    assert not got[:, np.setdiff1d(np.arange(cols), used)].any()
+    plain = [_Tree(t) for t in forest]
+    for i in sorted({0, rows - 1}):
+        ref = sum(_tree_shap(t, X[i], cols) for t in plain)
+        np.testing.assert_allclose(got[i, :-1], ref, rtol=0, atol=2e-5 * scale)
+
+
+@pytest.mark.parametrize("rows,cols,trees,depth", [(1, 3, 1, 1), (70, 12, 6, 5), (130, 300, 5, 7), (9, 5, 3, 16)])
+def test_contributions_by_table_and_by_walk(xgb, rows, cols, trees, depth):
+    """mgb_predict_contribs, which walks the tree records where the table or its
+    scratch would outgrow their bounds, agrees with the table."""
+    import ctypes
+
+    import device_lib as D
+    rng = np.random.default_rng(rows * 3 + cols)
+    bst, forest = _covered_forest(xgb, rng, cols, trees, depth)
+    X = rng.normal(size=(rows, cols)).astype(np.float32)
+    X[rng.random(X.shape) < 0.2] = np.nan
+    nodes, means, offsets = [], [], [0]
+    for t in forest:
+        n = np.zeros(len(t["left_children"]), D.TREE_NODE)
+        for key, source in (("left", "left_children"), ("right", "right_children"), ("feature", "split_indices"),
+                            ("threshold", "split_conditions"), ("leaf", "split_conditions"), ("cover", "sum_hessian"),
+                            ("default_left", "default_left")):
+            n[key] = t[source]
+        nodes.append(n)
+        means.append(_Tree(t).mean.astype(np.float32))
+        offsets.append(offsets[-1] + len(n))
+    dX, dn, dm = D.Device.of(X), D.Device.of(np.concatenate(nodes)), D.Device.of(np.concatenate(means))
+    do, out = D.Device.of(np.array(offsets, np.uint32)), D.Device(rows * (cols + 1) * 4)
+    D.check(D.lib().mgb_predict_contribs(dX.ptr, None, None, ctypes.c_uint32(rows), ctypes.c_uint32(cols), dn.ptr, dm.ptr,
+                                         do.ptr, ctypes.c_uint32(trees), ctypes.c_uint32(depth), ctypes.c_uint32(0),
+                                         ctypes.c_uint32(0), None, ctypes.c_float(0.25), out.ptr))
+    walk = out.read(np.float32, rows * (cols + 1)).reshape(rows, cols + 1)
+    table = bst.predict(xgb.DMatrix(X), pred_contribs=True)
+    scale = max(1.0, np.abs(table.astype(np.float64).sum(axis=1)).max())
+    np.testing.assert_allclose(walk, table, rtol=0, atol=4e-5 * scale)

@@ -330,11 +330,29 @@ __host__ __device__ constexpr uint32_t shap_words(uint32_t elements) {
 struct Quadrature {
   float t[kShapElements / 2], w[kShapElements / 2];
 };
+struct Points {
+  double t[kShapElements / 2];
+};
+
+// A feature's number in the table, the tiles' keys and the sums: its place
+// among the `count` features used (NULL: every feature, by itself); `count`
+// where it is not among them.
+__device__ __forceinline__ uint32_t used_slot(const uint32_t* __restrict__ used, uint32_t count, uint32_t feature) {
+  if (!used) return min(feature, count);
+  uint32_t lo = 0, hi = count;
+  while (lo < hi) {
+    const uint32_t mid = lo + (hi - lo) / 2;
+    if (used[mid] < feature) lo = mid + 1;
+    else hi = mid;
+  }
+  return lo < count && used[lo] == feature ? lo : count;
+}
 
 // One thread a leaf: walks up to the root, merging the tests of each feature.
 __global__ void k_shap_paths(const MgbTreeNode* __restrict__ nodes, const int64_t* __restrict__ parents,
-                             const uint32_t* __restrict__ leaves, uint32_t count, uint32_t elements, uint32_t cols,
-                             const double* __restrict__ points, uint32_t* __restrict__ table) {
+                             const uint32_t* __restrict__ leaves, uint32_t count, uint32_t elements,
+                             const uint32_t* __restrict__ used, uint32_t features, Points points,
+                             uint32_t* __restrict__ table) {
   for (uint64_t k = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; k < count; k += (uint64_t)gridDim.x * blockDim.x) {
     uint32_t feature[kShapElements], lo[kShapElements], hi[kShapElements], miss[kShapElements];
     double z[kShapElements];
@@ -366,10 +384,10 @@ __global__ void k_shap_paths(const MgbTreeNode* __restrict__ nodes, const int64_
     }
     for (uint32_t j = 0; j < elements; ++j) {
       uint32_t* e = rec + 1 + j * (3 + elements);
-      uint32_t f = cols, flag = 0, from = kMissingKey, span = kMissingKey;
+      uint32_t f = features, flag = 0, from = kMissingKey, span = kMissingKey;
       double share = 1.0;
       if (j < m) {
-        f = min(feature[j], cols);  // a feature the matrix lacks reads as missing
+        f = used_slot(used, features, feature[j]);  // a feature the matrix lacks reads as missing
         share = z[j];
         if (lo[j] >= hi[j]) {  // no number passes
           from = miss[j] ? kMissingKey : kMissingKey - 1u;
@@ -389,7 +407,7 @@ __global__ void k_shap_paths(const MgbTreeNode* __restrict__ nodes, const int64_
       e[1] = from;
       e[2] = span;
       for (uint32_t q = 0; q < elements / 2; ++q) {
-        const double t = points[q];
+        const double t = points.t[q];
         e[3 + q] = __float_as_uint((float)(share * (1.0 - t)));
         e[3 + elements / 2 + q] = __float_as_uint((float)((1.0 - share) / (share * (1.0 - t) + t)));
       }
@@ -402,40 +420,46 @@ __global__ void k_shap_paths(const MgbTreeNode* __restrict__ nodes, const int64_
 // row lacks.
 __global__ __launch_bounds__(256) void k_shap_keys(const float* __restrict__ X, const uint64_t* __restrict__ indptr,
                                                    const uint32_t* __restrict__ indices, uint32_t first, uint32_t rows,
-                                                   uint32_t cols, uint32_t* __restrict__ keys) {
+                                                   uint32_t cols, const uint32_t* __restrict__ used, uint32_t features,
+                                                   uint32_t* __restrict__ keys) {
   const uint32_t r0 = first + blockIdx.x * kWave;
-  uint32_t* tile = keys + (uint64_t)blockIdx.x * (cols + 1) * kWave;
+  uint32_t* tile = keys + (uint64_t)blockIdx.x * (features + 1) * kWave;
   if (!indptr) {
     // Lanes along the rows: a lane's reads of its row stay in the lines that
     // its neighbours' features share.
     const uint32_t r = min(r0 + threadIdx.x % kWave, rows - 1);
-    for (uint32_t f = threadIdx.x / kWave; f <= cols; f += blockDim.x / kWave)
-      tile[(uint64_t)f * kWave + threadIdx.x % kWave] = f < cols ? order_key(X[(uint64_t)r * cols + f]) : kMissingKey;
+    for (uint32_t f = threadIdx.x / kWave; f <= features; f += blockDim.x / kWave)
+      tile[(uint64_t)f * kWave + threadIdx.x % kWave] =
+          f < features ? order_key(X[(uint64_t)r * cols + (used ? used[f] : f)]) : kMissingKey;
     return;
   }
-  for (uint64_t i = threadIdx.x; i < (uint64_t)(cols + 1) * kWave; i += blockDim.x) tile[i] = kMissingKey;
+  for (uint64_t i = threadIdx.x; i < (uint64_t)(features + 1) * kWave; i += blockDim.x) tile[i] = kMissingKey;
   __syncthreads();
   for (uint32_t j = threadIdx.x / 4; j < kWave && r0 + j < rows; j += blockDim.x / 4)
-    for (uint64_t k = indptr[r0 + j] + threadIdx.x % 4; k < indptr[r0 + j + 1]; k += 4)
-      if (indices[k] < cols) tile[(uint64_t)indices[k] * kWave + j] = order_key(X[k]);
+    for (uint64_t k = indptr[r0 + j] + threadIdx.x % 4; k < indptr[r0 + j + 1]; k += 4) {
+      const uint32_t f = used_slot(used, features, indices[k]);
+      if (f < features) tile[(uint64_t)f * kWave + j] = order_key(X[k]);
+    }
 }
 
 struct ShapArgs {
   const uint32_t* table;
   const uint32_t* keys;     // k_shap_keys' tiles
   float* partial;           // per slice of the leaves: per tile, features x 64 rows
-  uint32_t leaves, cols, tiles;
+  uint32_t leaves, features, tiles;
   Quadrature quad;
 };
 
 // A wave holds 64 rows of one tile and takes a contiguous share of the leaves:
 // records come through scalar loads, the rows' keys from and their sums to LDS
 // (IN_LDS), where each wave has its own sums, added in wave order at the end;
-// matrices too wide for that keep both in memory, a partial to each wave.
+// more features than that holds keep both in memory, a partial to each wave.
 // Bound by vector operations, about 3 Q + 12 an element, and the chain of each
 // leaf's LDS sums.  5,000 x 32, 100 trees of depth 6: 0.137 ms, against 131.7
 // with a row a lane and the paths in scratch memory (LDS float atomics in the
-// place of load, add, store: 0.95 ms).
+// place of load, add, store: 0.95 ms).  In memory, whole calls against a row a
+// lane, 100 trees of depth 8: 1 row x 2,000 0.51 against 297 ms, 5,000 rows 21.8
+// against 774; 1 row x 100,000 CSR 1.4 against 296.
 constexpr uint32_t kShapWaves = 8;
 template <int M, bool IN_LDS>
 __global__ __launch_bounds__(kShapWaves * kWave) void k_contribs_paths(ShapArgs a) {
@@ -444,7 +468,7 @@ __global__ __launch_bounds__(kShapWaves * kWave) void k_contribs_paths(ShapArgs 
   extern __shared__ __align__(16) uint8_t shap_smem[];
   const uint32_t lane = threadIdx.x % kWave;
   const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), waves = blockDim.x / kWave;
-  const uint32_t tile = blockIdx.x, width = a.cols + 1;
+  const uint32_t tile = blockIdx.x, width = a.features + 1;
   const uint32_t slice = blockIdx.y * waves + wave, slices = gridDim.y * waves;
   const uint32_t* far_keys = a.keys + (uint64_t)tile * width * kWave;
   uint32_t* s_keys = reinterpret_cast<uint32_t*>(shap_smem);
@@ -519,29 +543,39 @@ __global__ __launch_bounds__(kShapWaves * kWave) void k_contribs_paths(ShapArgs 
   }
 }
 
-// out[r][f] from the partials in slice order, and the bias: the base margin
-// plus every tree's root mean.
-__global__ __launch_bounds__(256) void k_shap_finish(const float* __restrict__ partial, uint32_t slices,
-                                                     uint32_t tiles, uint32_t first, uint32_t rows, uint32_t cols,
-                                                     const float* __restrict__ root_means, uint32_t trees,
-                                                     const float* __restrict__ base, float base_value,
-                                                     float* __restrict__ out) {
-  const uint32_t width = cols + 1, tile = blockIdx.x;
-  const uint64_t stride = (uint64_t)tiles * width * kWave;
-  const float* src = partial + (uint64_t)tile * width * kWave;
-  const uint32_t r0 = first + tile * kWave;
-  for (uint32_t i = threadIdx.x; i < width * kWave; i += blockDim.x) {
-    const uint32_t j = i / width, f = i % width, r = r0 + j;
-    if (r >= rows || f == cols) continue;
+// out[r][f] from the partials in slice order, kFinishFeatures features of a
+// tile to a workgroup: lanes along the rows read, along the features write.
+// The bias, in the first of them: the base margin plus every tree's root mean.
+constexpr uint32_t kFinishFeatures = 16, kFinishThreads = 256;
+__global__ __launch_bounds__(kFinishThreads) void k_shap_finish(const float* __restrict__ partial, uint32_t partials,
+                                                                uint32_t tiles, uint32_t first, uint32_t rows,
+                                                                uint32_t cols, const uint32_t* __restrict__ used,
+                                                                uint32_t features,
+                                                                const float* __restrict__ root_means, uint32_t trees,
+                                                                const float* __restrict__ base, float base_value,
+                                                                float* __restrict__ out) {
+  __shared__ float sums[kFinishFeatures][kWave + 1];
+  const uint64_t width = (uint64_t)cols + 1;
+  const uint32_t tile = blockIdx.x, f0 = blockIdx.y * kFinishFeatures, r0 = first + tile * kWave;
+  const uint64_t stride = (uint64_t)tiles * (features + 1) * kWave;
+  const float* src = partial + (uint64_t)tile * (features + 1) * kWave;
+  const uint32_t here = f0 < features ? min(kFinishFeatures, features - f0) : 0u;
+  for (uint32_t i = threadIdx.x; i < here * kWave; i += kFinishThreads) {
     float sum = 0.0f;
-    for (uint32_t s = 0; s < slices; ++s) sum += src[s * stride + (uint64_t)f * kWave + j];
-    out[(uint64_t)r * width + f] = sum;
+#pragma unroll 4
+    for (uint32_t s = 0; s < partials; ++s) sum += src[s * stride + (uint64_t)f0 * kWave + i];
+    sums[i / kWave][i % kWave] = sum;
   }
-  if (threadIdx.x < kWave && r0 + threadIdx.x < rows) {
+  __syncthreads();
+  for (uint32_t i = threadIdx.x; i < kFinishFeatures * kWave; i += kFinishThreads) {
+    const uint32_t f = i % kFinishFeatures, r = r0 + i / kFinishFeatures;
+    if (f < here && r < rows) out[r * width + (used ? used[f0 + f] : f0 + f)] = sums[f][i / kFinishFeatures];
+  }
+  if (blockIdx.y == 0 && threadIdx.x < kWave && r0 + threadIdx.x < rows) {
     const uint32_t r = r0 + threadIdx.x;
     float bias = base ? base[r] : base_value;
     for (uint32_t t = 0; t < trees; ++t) bias += root_means[t];
-    out[(uint64_t)r * width + cols] = bias;
+    out[r * width + cols] = bias;
   }
 }
 
@@ -587,6 +621,56 @@ struct Scratch {
   ~Scratch() { if (p) (void)mgb_free(p); }
   int alloc(size_t bytes) { return mgb_malloc(&p, bytes ? bytes : 16); }
 };
+
+// How a call is split: workgroups of `waves` waves, `slices` shares of the
+// leaves to a tile, `chunk` tiles at a time with `partials` sums each.
+struct ShapPlan {
+  bool in_lds;
+  uint32_t waves;
+  uint64_t slices, partials, tile_bytes, chunk;
+};
+
+// Keys and sums of a chunk stay within this: they come from the allocator's
+// kept blocks call after call.
+constexpr uint64_t kShapScratch = uint64_t(256) << 20;
+
+// False where a tile's keys and one partial alone are more, and where so many
+// tiles meet so few partials (a wave to each) that a row a lane over the tree
+// records takes less time.  Table against walk, CSR rows, trees of depth 8: 30,393
+// features used (34 blocks), 94 tiles 0.92 against 1.26 s, 250 tiles 2.28
+// against 2.13; 11,396 (92 blocks), 313 tiles 0.68 against 0.97, 750 tiles 1.68
+// against 1.84; 2,000 (511), 1,563 tiles 0.40 against 1.52.
+constexpr uint64_t kShapFewBlocks = 64, kShapTilesABlock = 6, kShapFewTiles = 4;
+bool shap_plan(const MgbShap& p, ShapPlan& plan) {
+  const uint64_t tile_bytes = ((uint64_t)p.features + 1) * kWave * sizeof(float);
+  const uint64_t blocks = kShapScratch / tile_bytes;  // tiles' keys and partials that fit
+  const uint64_t all_tiles = ((uint64_t)p.rows + kWave - 1) / kWave;
+  if (blocks < 2 || (blocks < kShapFewBlocks && all_tiles > kShapTilesABlock * blocks)) return false;
+  // LDS: the tile's keys and each wave's sums.  One wave there, or two where
+  // there are tiles enough, is slower than four with both in memory: 290
+  // features, 100 trees of depth 6, 1 / 5,000 rows 0.50 / 3.74 against 0.29 /
+  // 1.24 ms; 128 features (two waves) 0.19 / 1.19 against 0.24 / 0.57, 1,000 rows
+  // 0.42 against 0.22.
+  uint32_t waves = kShapWaves;
+  while (waves > 1 && (waves + 1) * tile_bytes > 150 * 1024) waves /= 2;
+  plan.in_lds = waves > 2 || (waves == 2 && all_tiles <= kShapFewTiles);
+  if (!plan.in_lds) {
+    waves = 4;  // a partial to each
+    while (waves > 1 && waves + 1 > blocks) waves /= 2;
+  }
+  const uint64_t each = plan.in_lds ? 1 : waves;  // partials of a slice
+  // Slices of the leaves: enough waves for the chip, some leaves to each, and
+  // no more than one tile's scratch has room for.
+  uint64_t slices = std::max<uint64_t>(1, 4096 / (all_tiles * waves));
+  slices = std::min<uint64_t>(slices, p.leaves / (8ull * waves));
+  slices = std::max<uint64_t>(1, std::min<uint64_t>(slices, (blocks - 1) / each));
+  plan.waves = waves;
+  plan.slices = slices;
+  plan.partials = slices * each;
+  plan.tile_bytes = tile_bytes;
+  plan.chunk = std::min<uint64_t>(all_tiles, blocks / (1 + plan.partials));
+  return true;
+}
 
 uint32_t explain_grid(uint64_t rows, uint32_t block) {
   uint64_t g = (rows + block - 1) / block;
@@ -653,22 +737,27 @@ size_t mgb_shap_table_bytes(uint32_t leaves, uint32_t elements) {
 }
 
 int mgb_shap_paths(const MgbTreeNode* nodes, const int64_t* parents, const uint32_t* leaves, uint32_t count,
-                   uint32_t elements, uint32_t cols, uint32_t* table) {
+                   uint32_t elements, const uint32_t* used, uint32_t features, uint32_t* table) {
   if (elements < 2 || elements > kShapElements || elements % 2) {
     set_error("mgb_shap_paths: elements must be even, 2 to " + std::to_string(kShapElements));
     return -1;
   }
   if (!count) return 0;
   if (!nodes || !parents || !leaves || !table) { set_error("mgb_shap_paths: null argument"); return -1; }
-  if (cols >= (1u << 24)) { set_error("mgb_shap_paths: 2^24 features or more"); return -1; }
-  double t[kShapElements / 2], w[kShapElements / 2];
-  gauss_legendre(elements / 2, t, w);
-  Scratch points;
-  if (points.alloc(sizeof(t)) || mgb_memcpy_h2d_async(points.p, t, sizeof(t))) return -1;
+  if (features >= (1u << 24)) { set_error("mgb_shap_paths: 2^24 features or more"); return -1; }
+  Points points;
+  double w[kShapElements / 2];
+  gauss_legendre(elements / 2, points.t, w);
   launch(MGB_PROF_PREDICT, k_shap_paths, dim3(explain_grid(count, 64)), dim3(64), 0, nodes, parents, leaves, count,
-         elements, cols, (const double*)points.p, table);
+         elements, used, features, points, table);
   MGB_LAUNCH_CHECK("k_shap_paths");
   return 0;
+}
+
+size_t mgb_shap_scratch_bytes(const MgbShap* p) {
+  ShapPlan plan;
+  if (!p || !p->rows || !shap_plan(*p, plan)) return 0;
+  return plan.chunk * plan.tile_bytes * (1 + plan.partials);
 }
 
 int mgb_predict_shap(const MgbShap* p) {
@@ -678,59 +767,58 @@ int mgb_predict_shap(const MgbShap* p) {
     set_error("mgb_predict_shap: null argument");
     return -1;
   }
-  if (p->elements < 2 || p->elements > kShapElements || p->elements % 2 || p->cols >= (1u << 24)) {
-    set_error("mgb_predict_shap: elements must be even, 2 to " + std::to_string(kShapElements) +
-              ", and features below 2^24");
+  if (p->elements < 2 || p->elements > kShapElements || p->elements % 2) {
+    set_error("mgb_predict_shap: elements must be even, 2 to " + std::to_string(kShapElements));
+    return -1;
+  }
+  if (p->features > p->cols || (!p->used && p->features != p->cols)) {
+    set_error("mgb_predict_shap: features must be the matrix's columns, or fewer and listed in used");
+    return -1;
+  }
+  ShapPlan plan;
+  if (!shap_plan(*p, plan)) {
+    set_error("mgb_predict_shap: too many features or rows for the scratch (mgb_shap_scratch_bytes)");
     return -1;
   }
   ShapArgs a{};
   a.table = p->table;
   a.leaves = p->leaves;
-  a.cols = p->cols;
+  a.features = p->features;
   double t[kShapElements / 2], w[kShapElements / 2];
   gauss_legendre(p->elements / 2, t, w);
   for (uint32_t q = 0; q < p->elements / 2; ++q) { a.quad.t[q] = (float)t[q]; a.quad.w[q] = (float)w[q]; }
-  // LDS: the tile's keys and each wave's sums.
-  const uint64_t tile_bytes = ((uint64_t)p->cols + 1) * kWave * sizeof(float);
-  uint32_t waves = kShapWaves;
-  while (waves > 1 && (waves + 1) * tile_bytes > 150 * 1024) waves /= 2;
-  const bool in_lds = (waves + 1) * tile_bytes <= 150 * 1024;
-  if (!in_lds) waves = 4;
-  // Slices of the leaves: enough waves for the chip, some leaves to each.
-  const uint64_t all_tiles = ((uint64_t)p->rows + kWave - 1) / kWave;
-  uint64_t slices = std::max<uint64_t>(1, 4096 / (all_tiles * waves));
-  slices = std::max<uint64_t>(1, std::min<uint64_t>(slices, p->leaves / (8ull * waves)));
-  const uint64_t partials = in_lds ? slices : slices * waves;
-  // Row chunks whose keys and partials stay within 256 MB.
-  const uint64_t chunk = std::min<uint64_t>(
-      all_tiles, std::max<uint64_t>(1, (uint64_t(256) << 20) / (tile_bytes * (1 + partials))));
   Scratch keys, partial;
-  if (keys.alloc(chunk * tile_bytes) || partial.alloc(chunk * tile_bytes * partials)) return -1;
-  for (uint64_t at = 0; at < all_tiles; at += chunk) {
-    const uint32_t tiles = (uint32_t)std::min<uint64_t>(chunk, all_tiles - at);
+  if (keys.alloc(plan.chunk * plan.tile_bytes) || partial.alloc(plan.chunk * plan.tile_bytes * plan.partials)) return -1;
+  // Columns that no split names.
+  if (p->features < p->cols && mgb_fill_f32(p->out, (uint64_t)p->rows * ((uint64_t)p->cols + 1), 0.0f)) return -1;
+  const uint64_t all_tiles = ((uint64_t)p->rows + kWave - 1) / kWave;
+  for (uint64_t at = 0; at < all_tiles; at += plan.chunk) {
+    const uint32_t tiles = (uint32_t)std::min<uint64_t>(plan.chunk, all_tiles - at);
     const uint32_t first = (uint32_t)(at * kWave);
     a.keys = (const uint32_t*)keys.p;
     a.partial = (float*)partial.p;
     a.tiles = tiles;
     launch(MGB_PROF_PREDICT, k_shap_keys, dim3(tiles), dim3(256), 0, p->X, p->indptr, p->indices, first, p->rows,
-           p->cols, (uint32_t*)keys.p);
+           p->cols, p->used, p->features, (uint32_t*)keys.p);
     MGB_LAUNCH_CHECK("k_shap_keys");
-    const dim3 grid(tiles, (uint32_t)slices);
-    const uint32_t lds = (uint32_t)((waves + 1) * tile_bytes);
+    const dim3 grid(tiles, (uint32_t)plan.slices);
+    const uint32_t lds = plan.in_lds ? (uint32_t)((plan.waves + 1) * plan.tile_bytes) : 0;
     int status = -1;
     switch (p->elements) {
-      case 2: status = launch_paths<2>(a, in_lds, grid, waves, lds); break;
-      case 4: status = launch_paths<4>(a, in_lds, grid, waves, lds); break;
-      case 6: status = launch_paths<6>(a, in_lds, grid, waves, lds); break;
-      case 8: status = launch_paths<8>(a, in_lds, grid, waves, lds); break;
-      case 10: status = launch_paths<10>(a, in_lds, grid, waves, lds); break;
-      case 12: status = launch_paths<12>(a, in_lds, grid, waves, lds); break;
-      case 14: status = launch_paths<14>(a, in_lds, grid, waves, lds); break;
-      case 16: status = launch_paths<16>(a, in_lds, grid, waves, lds); break;
+      case 2: status = launch_paths<2>(a, plan.in_lds, grid, plan.waves, lds); break;
+      case 4: status = launch_paths<4>(a, plan.in_lds, grid, plan.waves, lds); break;
+      case 6: status = launch_paths<6>(a, plan.in_lds, grid, plan.waves, lds); break;
+      case 8: status = launch_paths<8>(a, plan.in_lds, grid, plan.waves, lds); break;
+      case 10: status = launch_paths<10>(a, plan.in_lds, grid, plan.waves, lds); break;
+      case 12: status = launch_paths<12>(a, plan.in_lds, grid, plan.waves, lds); break;
+      case 14: status = launch_paths<14>(a, plan.in_lds, grid, plan.waves, lds); break;
+      case 16: status = launch_paths<16>(a, plan.in_lds, grid, plan.waves, lds); break;
     }
     if (status) return -1;
-    launch(MGB_PROF_PREDICT, k_shap_finish, dim3(tiles), dim3(256), 0, (const float*)partial.p, (uint32_t)partials,
-           tiles, first, p->rows, p->cols, p->root_means, p->trees, p->base, p->base_value, p->out);
+    const dim3 finish(tiles, std::max(1u, (p->features + kFinishFeatures - 1) / kFinishFeatures));
+    launch(MGB_PROF_PREDICT, k_shap_finish, finish, dim3(kFinishThreads), 0, (const float*)partial.p,
+           (uint32_t)plan.partials, tiles, first, p->rows, p->cols, p->used, p->features, p->root_means, p->trees,
+           p->base, p->base_value, p->out);
     MGB_LAUNCH_CHECK("k_shap_finish");
   }
   return 0;

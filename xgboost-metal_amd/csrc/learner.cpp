@@ -1185,12 +1185,18 @@ uint32_t node_means(const std::vector<MgbTreeNode>& t, float* means) {
 }  // namespace
 
 // The path table of trees [0, end), laid out on the device from the uploaded
-// nodes.
-void Learner::build_paths(uint32_t end) {
-  if (shap_trees_ == end) return;
+// nodes; false: it would outgrow kShapTableBytes.  Up to kShapAllFeatures
+// columns, whose keys and sums a workgroup of eight waves holds in LDS, the
+// table takes every feature by its own number; beyond, those that some split
+// names (a model of many columns uses few of them).
+bool Learner::build_paths(uint32_t end) {
+  constexpr uint32_t kShapAllFeatures = 64;
+  constexpr size_t kShapTableBytes = size_t(16) << 30;
+  if (shap_trees_ == end) return true;
   shap_trees_ = SIZE_MAX;
   std::vector<int64_t> parents;
-  std::vector<uint32_t> leaves;
+  std::vector<uint32_t> leaves, used;
+  const bool all = num_feature <= kShapAllFeatures;
   std::vector<float> roots, means;
   uint32_t deepest = 0;
   for (uint32_t t = 0; t < end; ++t) {
@@ -1204,6 +1210,7 @@ void Learner::build_paths(uint32_t end) {
       if (nodes[i].left < 0) continue;
       parents[at + nodes[i].left] = (int64_t)(at + i) * 2 + 1;
       parents[at + nodes[i].right] = (int64_t)(at + i) * 2;
+      if (!all && (uint32_t)nodes[i].feature < num_feature) used.push_back((uint32_t)nodes[i].feature);
     }
     // Nodes that no split names are not part of the tree.
     for (size_t i = 0; i < nodes.size(); ++i)
@@ -1211,6 +1218,15 @@ void Learner::build_paths(uint32_t end) {
   }
   const uint32_t elements = mgb_shap_elements(deepest);
   require(elements != 0, "mgb_predict_contribs: exact contributions need trees of depth at most 16");
+  if (mgb_shap_table_bytes((uint32_t)leaves.size(), elements) > kShapTableBytes) return false;
+  std::sort(used.begin(), used.end());
+  used.erase(std::unique(used.begin(), used.end()), used.end());
+  shap_features_ = all ? num_feature : (uint32_t)used.size();
+  d_shap_used_.release();
+  if (!all) {
+    d_shap_used_.ensure(std::max<size_t>(used.size(), 1) * sizeof(uint32_t));
+    d_shap_used_.upload(used.data(), used.size() * sizeof(uint32_t));
+  }
   if (parents.empty()) parents.push_back(-1);
   DeviceBuffer d_parents, d_leaves;
   d_parents.upload(parents.data(), parents.size() * sizeof(int64_t));
@@ -1220,11 +1236,13 @@ void Learner::build_paths(uint32_t end) {
   d_root_means_.upload(roots.data(), roots.size() * sizeof(float));
   d_shap_table_.ensure(mgb_shap_table_bytes((uint32_t)leaves.size(), elements));
   kcheck(mgb_shap_paths(d_model_nodes_.as<MgbTreeNode>(), d_parents.as<int64_t>(), d_leaves.as<uint32_t>(),
-                        (uint32_t)leaves.size(), elements, num_feature, d_shap_table_.as<uint32_t>()),
+                        (uint32_t)leaves.size(), elements, d_shap_used_.as<uint32_t>(), shap_features_,
+                        d_shap_table_.as<uint32_t>()),
          "paths");
   shap_leaves_ = (uint32_t)leaves.size();
   shap_elements_ = elements;
   shap_trees_ = end;
+  return true;
 }
 
 std::vector<float> Learner::predict_explain(DMatrix& data, int type, uint32_t end) {
@@ -1247,31 +1265,34 @@ std::vector<float> Learner::predict_explain(DMatrix& data, int type, uint32_t en
   const uint64_t* indptr = data.sparse ? data.d_indptr.as<uint64_t>() : nullptr;
   const uint32_t* indices = data.sparse ? data.d_indices.as<uint32_t>() : nullptr;
   const float* X = data.sparse ? data.d_values.as<float>() : data.d_data.as<float>();
-  if (type == 6) {
-    kcheck(mgb_predict_leaf(X, indptr, indices, data.rows, data.cols, d_model_nodes_.as<MgbTreeNode>(),
-                            d_model_offsets_.as<uint32_t>(), end, d_out.as<float>()),
-           "leaf prediction");
-  } else if (type == 2 && data.cols < (1u << 24)) {
-    build_paths(end);
-    DeviceBuffer d_base;
-    if (!data.base_margin.empty()) {
-      require(data.base_margin.size() == data.rows, "base_margin must have one value per row.");
-      d_base.upload(data.base_margin.data(), data.rows * sizeof(float));
-    }
-    MgbShap p{};
+  MgbShap p{};
+  if (type == 2 && build_paths(end)) {
     p.X = X;
     p.indptr = indptr;
     p.indices = indices;
     p.table = d_shap_table_.as<uint32_t>();
+    p.used = d_shap_used_.as<uint32_t>();
     p.root_means = d_root_means_.as<float>();
-    p.base = d_base.get() ? d_base.as<float>() : nullptr;
     p.out = d_out.as<float>();
     p.rows = data.rows;
     p.cols = data.cols;
     p.leaves = shap_leaves_;
     p.elements = shap_elements_;
     p.trees = end;
+    p.features = p.used ? shap_features_ : data.cols;
     p.base_value = base_margin_value();
+  }
+  if (type == 6) {
+    kcheck(mgb_predict_leaf(X, indptr, indices, data.rows, data.cols, d_model_nodes_.as<MgbTreeNode>(),
+                            d_model_offsets_.as<uint32_t>(), end, d_out.as<float>()),
+           "leaf prediction");
+  } else if (type == 2 && mgb_shap_scratch_bytes(&p) != 0) {
+    DeviceBuffer d_base;
+    if (!data.base_margin.empty()) {
+      require(data.base_margin.size() == data.rows, "base_margin must have one value per row.");
+      d_base.upload(data.base_margin.data(), data.rows * sizeof(float));
+    }
+    p.base = d_base.get() ? d_base.as<float>() : nullptr;
     kcheck(mgb_predict_shap(&p), "contribution prediction");
   } else {
     std::vector<float> means;

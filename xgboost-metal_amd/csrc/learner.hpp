@@ -215,11 +215,12 @@ class Learner {
   // Model on the device for prediction.
   DeviceBuffer d_model_nodes_, d_model_offsets_;
   DeviceBuffer d_model_means_;  // each node's cover-weighted mean leaf value (contributions)
-  // Path table of trees [0, shap_trees_) for exact contributions (SIZE_MAX: none).
-  void build_paths(uint32_t end);
+  // Path table of trees [0, shap_trees_) for exact contributions (SIZE_MAX:
+  // none), over shap_features_ features: those of d_shap_used_, or all.
+  bool build_paths(uint32_t end);
   size_t shap_trees_ = SIZE_MAX;
-  uint32_t shap_leaves_ = 0, shap_elements_ = 0;
-  DeviceBuffer d_shap_table_, d_root_means_;
+  uint32_t shap_leaves_ = 0, shap_elements_ = 0, shap_features_ = 0;
+  DeviceBuffer d_shap_table_, d_shap_used_, d_root_means_;
   size_t model_version_ = SIZE_MAX, model_trees_ = 0;
   size_t uploaded_trees_ = 0;
   // The trees packed for prediction, on the host and (the first
