@@ -363,7 +363,9 @@ typedef struct {
  * leaf a tree, added in tree order.  X: rows x cols floats, or with indptr and
  * indices a CSR matrix's `entries` values (column indices strictly increasing
  * within a row; absent entries and NaN follow default_left).  cols is the
- * model's feature count; depth the deepest tree's.  base may be out. */
+ * model's feature count; depth the deepest tree's and steps the sum of the
+ * trees' depths (which kernel is the faster depends on them, no result does).
+ * base may be out. */
 typedef struct {
   const float* X;
   const uint64_t* indptr;
@@ -372,7 +374,7 @@ typedef struct {
   const uint32_t* offsets;
   const float* base;
   float* out;
-  uint64_t entries;
+  uint64_t entries, steps;
   uint32_t rows, cols, trees, depth, objective;
   float base_value;
 } MgbPredict;

@@ -258,3 +258,47 @@ def test_fits_with_leaves_of_zero(xgb, rows):
         np.testing.assert_array_equal(bst.inplace_predict(X), expect)
     zeros = json.loads(fits[0].save_raw("json"))["learner"]["gradient_booster"]["model"]["trees"][-1]
     assert any(l < 0 and v == 0 for l, v in zip(zeros["left_children"], zeros["split_conditions"]))
+
+
+def _chain(rng, cols, depth):
+    """A tree whose every right child is split again, `depth` levels down."""
+    n = 2 * depth + 1
+    inner = [0] + [2 * d for d in range(1, depth)]
+    left, right = [-1] * n, [-1] * n
+    for d, k in enumerate(inner):
+        left[k], right[k] = 2 * d + 1, 2 * d + 2
+    cond = [float(np.float32(-1.0 - rng.random())) if left[k] >= 0 else float(np.float32(rng.normal())) for k in range(n)]
+    parents = [2147483647] + [0] * (n - 1)
+    for k in inner:
+        parents[left[k]] = parents[right[k]] = k
+    return {"left_children": left, "right_children": right, "split_indices": [int(f) for f in rng.integers(cols, size=n)],
+            "split_conditions": cond, "default_left": [0] * n, "parents": parents, "loss_changes": [0] * n,
+            "sum_hessian": [0] * n, "base_weights": [0] * n}
+
+
+@pytest.mark.parametrize("rows,cols,trees,depth,chain", [
+    (1, 5, 1, 8, 0), (63, 5, 1, 9, 0), (65, 9, 2, 4, 0), (12289, 9, 1, 6, 0), (32767, 120, 2, 4, 0), (32768, 120, 2, 4, 0),
+    (40000, 120, 3, 3, 0), (33000, 1200, 8, 6, 0), (33000, 1200, 9, 6, 0), (13000, 6, 30, 3, 150), (300, 6, 30, 3, 150),
+    (32769, 6, 3, 3, 500), (12300, 6, 1, 3, 3000)])
+def test_margins_where_rows_take_few_or_uneven_steps(xgb, rows, cols, trees, depth, chain):
+    """Both sides of the limits of the row-a-lane kernel: few steps a row, wide
+    rows of some steps, one tree much deeper than the others."""
+    import scipy.sparse as sp
+    rng = np.random.default_rng(rows + cols + trees)
+    forest = [_random_tree(rng, cols, depth, False) for _ in range(trees)]
+    if chain:
+        forest.insert(1, _chain(rng, cols, chain))
+    X = _values(rng, rows, cols, 0.15)
+    _special_values(rng, forest[:1] if chain else forest, X)
+    bst = _booster(xgb, forest, cols)
+    base = rng.normal(size=rows).astype(np.float32)
+    expect = _margins(forest, X, base)
+    _same_bits(bst.predict(xgb.DMatrix(X, base_margin=base)), expect)
+    keep = np.arange(rows) if cols <= 120 else np.arange(7000)
+    r, c = np.nonzero(~np.isnan(X[keep]))
+    csr = sp.csr_matrix((X[r, c], (r, c)), shape=(len(keep), cols))
+    _same_bits(bst.predict(xgb.DMatrix(csr, base_margin=base[keep])), expect[keep])
+    _same_bits(bst.predict(xgb.DMatrix(X), iteration_range=(0, 1)), _margins(forest[:1], X, 0.25))
+    logistic = _booster(xgb, forest, cols, "binary:logistic")
+    margin = logistic.predict(xgb.DMatrix(X), output_margin=True).astype(np.float64)
+    np.testing.assert_allclose(logistic.predict(xgb.DMatrix(X)), 1.0 / (1.0 + np.exp(-margin)), rtol=4e-7, atol=0)

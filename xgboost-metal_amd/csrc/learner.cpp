@@ -515,9 +515,11 @@ bool Learner::pack_model() {
   if (num_feature >= MGB_PACKED_FEATURES) return false;
   const size_t had = packed_offsets_.size() - 1;
   while (packed_fits_ && packed_offsets_.size() <= trees.size()) {
+    uint32_t depth = 0;
     packed_fits_ = packed_nodes_.size() + trees[packed_offsets_.size() - 1].nodes.size() < UINT32_MAX &&
-                   pack_tree(trees[packed_offsets_.size() - 1].nodes, num_feature, packed_nodes_, packed_depth_);
+                   pack_tree(trees[packed_offsets_.size() - 1].nodes, num_feature, packed_nodes_, depth);
     packed_offsets_.push_back((uint32_t)packed_nodes_.size());
+    packed_depths_.push_back(depth);
   }
   if (!packed_fits_) return false;
   if (packed_offsets_.size() - 1 == had && packed_uploaded_ == packed_nodes_.size()) return true;
@@ -563,7 +565,10 @@ void Learner::predict_into(DMatrix& data, uint32_t begin, uint32_t end, bool tra
     p.rows = data.rows;
     p.cols = data.cols;
     p.trees = end - begin;
-    p.depth = packed_depth_;
+    for (uint32_t t = begin; t < end; ++t) {
+      p.depth = std::max(p.depth, packed_depths_[t]);
+      p.steps += packed_depths_[t];
+    }
     p.objective = transform ? (uint32_t)objective() : 0u;
     kcheck(mgb_predict_packed(&p), "prediction");
     return;
@@ -1586,7 +1591,7 @@ void Learner::load_model(const Json& input) {
   model_version_ = SIZE_MAX;
   packed_nodes_.clear();
   packed_offsets_.assign(1, 0);
-  packed_depth_ = 0;
+  packed_depths_.clear();
   packed_fits_ = true;
   packed_uploaded_ = 0;
   shap_trees_ = SIZE_MAX;

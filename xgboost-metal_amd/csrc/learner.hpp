@@ -227,7 +227,7 @@ class Learner {
   // packed_uploaded_ nodes) on the device.
   std::vector<MgbPackedNode> packed_nodes_;
   std::vector<uint32_t> packed_offsets_{0};
-  uint32_t packed_depth_ = 0;
+  std::vector<uint32_t> packed_depths_;
   bool packed_fits_ = true;
   size_t packed_uploaded_ = 0;
   DeviceBuffer d_packed_nodes_, d_packed_offsets_;

@@ -9,7 +9,8 @@
 // leaf's distance is 0, its feature is one past the model's features -- no row
 // has it, so it reads as missing -- and its default is left, where 0 is below
 // its word: a walk that has reached a leaf stays there, and every row takes the
-// same number of steps, the deepest tree's depth, with no exit test.
+// same number of steps, the deepest tree's depth, with no exit test (but in
+// k_predict_rows).
 //
 // Values are compared as order keys (order_key): NaN's key is the
 // largest word, a split node's word is its threshold's key plus its
@@ -334,6 +335,38 @@ __global__ __launch_bounds__(kStageWaves * kWave) void k_predict_staged(PredictA
   if (slice == 0 && r < nr) a.out[r0 + r] = finish(a, sum);
 }
 
+// A row's keys where its values lie in memory.
+template <bool SPARSE>
+struct FarRow {
+  const float* values;
+  const uint32_t* indices;  // CSR: the row's columns
+  uint32_t entries, cols;
+  __device__ __forceinline__ FarRow(const PredictArgs& a, uint64_t r) : cols(a.cols) {
+    if constexpr (SPARSE) {
+      const uint64_t b = a.indptr[r];
+      values = a.X + b;
+      indices = a.indices + b;
+      entries = (uint32_t)(a.indptr[r + 1] - b);
+    } else {
+      values = a.X + r * a.cols;
+    }
+  }
+  __device__ __forceinline__ uint32_t operator()(uint32_t f) const {
+    if (f >= cols) return kMissingKey;
+    if constexpr (SPARSE) {
+      uint32_t lo = 0, hi = entries;
+      while (lo < hi) {
+        const uint32_t mid = lo + (hi - lo) / 2;
+        if (indices[mid] < f) lo = mid + 1;
+        else hi = mid;
+      }
+      return lo < entries && indices[lo] == f ? order_key(values[lo]) : kMissingKey;
+    } else {
+      return order_key(values[f]);
+    }
+  }
+};
+
 // Few rows, or rows too wide for LDS: a wave to a row, a lane to a tree, two
 // trees side by side; the wave adds its 64 leaves in tree order.  A chain of
 // depth x 2 memory round trips: 16 rows x 32, 100 trees of depth 6, 236 -> 8.5
@@ -351,26 +384,7 @@ __global__ __launch_bounds__(kDirectWaves * kWave) void k_predict_direct(Predict
   const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   const uint32_t waves = blockDim.x / kWave;
   for (uint64_t r = (uint64_t)blockIdx.x * waves + wave; r < a.rows; r += (uint64_t)gridDim.x * waves) {
-    const float* row = SPARSE ? a.X : a.X + r * a.cols;
-    uint64_t b = 0, e = 0;
-    if constexpr (SPARSE) {
-      b = a.indptr[r];
-      e = a.indptr[r + 1];
-    }
-    auto key_of = [&](uint32_t f) -> uint32_t {
-      if (f >= a.cols) return kMissingKey;
-      if constexpr (SPARSE) {
-        uint64_t lo = b, hi = e;
-        while (lo < hi) {
-          const uint64_t mid = lo + (hi - lo) / 2;
-          if (a.indices[mid] < f) lo = mid + 1;
-          else hi = mid;
-        }
-        return lo < e && a.indices[lo] == f ? order_key(row[lo]) : kMissingKey;
-      } else {
-        return order_key(row[f]);
-      }
-    };
+    const FarRow<SPARSE> row(a, r);
     float sum = a.base ? a.base[r] : a.base_value;
     for (uint32_t t0 = 0; t0 < a.trees; t0 += 2 * kWave) {
       uint2 n[2];
@@ -384,7 +398,7 @@ __global__ __launch_bounds__(kDirectWaves * kWave) void k_predict_direct(Predict
       for (uint32_t d = 0; d < a.depth; ++d) {
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
-          at[j] += packed_step(n[j].x, n[j].y, key_of(packed_feature(n[j].y)));
+          at[j] += packed_step(n[j].x, n[j].y, row(packed_feature(n[j].y)));
           n[j] = a.nodes[at[j]];
         }
       }
@@ -399,8 +413,43 @@ __global__ __launch_bounds__(kDirectWaves * kWave) void k_predict_direct(Predict
   }
 }
 
+// Few steps a row, or a few trees much deeper than the others: a row a lane,
+// each tree left at its leaf (a split's distance is never 0).  Bound by the
+// chain of node and value loads, which grows with the steps (the trees' depths
+// added up) where the other two kernels' times hardly do; those read whole
+// rows, or give a row a wave, whatever the trees, and walk every tree for the
+// deepest one's steps.  Whole calls, this kernel against the other, us:
+// - one tree of depth 6: 12,000 x 64 33 / 40, 1M x 8 493 / 510, CSR 200,000 x 2,000
+//   115 / 130, 64 rows 29 to 33 / 30 to 33; two: 1,000 x 64 33 / 32, 100,000 x 64 71 / 65;
+// - staged rows of many columns: 100,000 x 400, 24 steps 93 / 120, 48 131 / 131,
+//   96 176 / 124; 1M x 128, 6 steps 593 / 681, 12 685 / 666 (13,000 x 400, 24: 42 / 41);
+// - rows too wide for LDS: 200,000 x 20,000 CSR, 48 steps 295 / 455, 96 431 / 372;
+//   100,000 x 1,200 138 / 179, 207 / 192 (13,000 x 1,200, 48: 61 / 46);
+// - one tree of depth 200 among 99 of depth 6 (20,000 steps for 794): 200,000 x 32
+//   676 / 1,685, 13,000 226 / 289; among nine (2,000 for 254) 276 / 287, 90 / 128.
+constexpr uint32_t kRowThreads = 64;
+constexpr uint32_t kRowsSteps = 8, kRowsFarSteps = 48, kRowsColumns = 14, kRowsDepths = 12;
+constexpr uint32_t kRowsMany = 32768;
 template <bool SPARSE>
-int predict_packed(PredictArgs a, uint64_t entries) {
+__global__ __launch_bounds__(kRowThreads) void k_predict_rows(PredictArgs a) {
+  for (uint64_t r = (uint64_t)blockIdx.x * kRowThreads + threadIdx.x; r < a.rows; r += (uint64_t)gridDim.x * kRowThreads) {
+    const FarRow<SPARSE> row(a, r);
+    float sum = a.base ? a.base[r] : a.base_value;
+    for (uint32_t t = 0; t < a.trees; ++t) {
+      uint32_t at = a.offsets[t];
+      uint2 n = a.nodes[at];
+      while (n.y & 0xffffu) {
+        at += packed_step(n.x, n.y, row(packed_feature(n.y)));
+        n = a.nodes[at];
+      }
+      sum = sum + packed_leaf(n.x);
+    }
+    a.out[r] = finish(a, sum);
+  }
+}
+
+template <bool SPARSE>
+int predict_packed(PredictArgs a, uint64_t entries, uint64_t steps) {
   const size_t cell = SPARSE ? sizeof(uint2) : sizeof(uint32_t);
   // A row's store in LDS: its keys and the leaves' feature, or its presence
   // words; an odd stride spreads the rows over the banks.
@@ -412,7 +461,17 @@ int predict_packed(PredictArgs a, uint64_t entries) {
   const uint64_t budget = kLdsBytes - (kOffsetWindow + 8) * sizeof(uint32_t) - tree_lds;
   const uint32_t fit = (uint32_t)std::min<uint64_t>(kStageWaves, budget / tile_bytes);  // 64-row tiles
   const uint32_t direct_rows = SPARSE ? kDirectRowsCsr : kDirectRows;
-  if (a.rows < direct_rows || fit == 0 || a.cols == 0) {
+  const bool staged = a.rows >= direct_rows && fit != 0;
+  const bool many = a.rows >= kRowsMany;
+  if (steps <= kRowsSteps || (many && !staged && steps <= kRowsFarSteps) ||
+      (many && staged && !SPARSE && steps * kRowsColumns <= a.cols) ||
+      (staged && (uint64_t)a.trees * a.depth > kRowsDepths * steps)) {
+    const uint32_t grid = (uint32_t)std::min<uint64_t>(((uint64_t)a.rows + kRowThreads - 1) / kRowThreads, 1u << 20);
+    launch(MGB_PROF_PREDICT, k_predict_rows<SPARSE>, dim3(grid), dim3(kRowThreads), 0, a);
+    MGB_LAUNCH_CHECK("k_predict_rows");
+    return 0;
+  }
+  if (!staged || a.cols == 0) {
     const uint32_t waves = a.rows < direct_rows ? 1 : kDirectWaves;
     const uint32_t grid = (uint32_t)std::min<uint64_t>(((uint64_t)a.rows + waves - 1) / waves, 16384);
     launch(MGB_PROF_PREDICT, k_predict_direct<SPARSE>, dim3(grid), dim3(waves * kWave), 0, a);
@@ -474,7 +533,7 @@ int mgb_predict_packed(const MgbPredict* p) {
   a.rows = p->rows; a.cols = p->cols; a.trees = p->trees; a.depth = p->depth;
   a.transform = p->objective == 1 ? 1u : 0u;
   a.base_value = p->base_value;
-  return p->indptr ? predict_packed<true>(a, p->entries) : predict_packed<false>(a, 0);
+  return p->indptr ? predict_packed<true>(a, p->entries, p->steps) : predict_packed<false>(a, 0, p->steps);
 }
 
 }  // extern "C"
