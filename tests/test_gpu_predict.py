@@ -277,8 +277,8 @@ def _chain(rng, cols, depth):
 
 
 @pytest.mark.parametrize("rows,cols,trees,depth,chain", [
-    (1, 5, 1, 8, 0), (63, 5, 1, 9, 0), (65, 9, 2, 4, 0), (12289, 9, 1, 6, 0), (32767, 120, 2, 4, 0), (32768, 120, 2, 4, 0),
-    (40000, 120, 3, 3, 0), (33000, 1200, 8, 6, 0), (33000, 1200, 9, 6, 0), (13000, 6, 30, 3, 150), (300, 6, 30, 3, 150),
+    (1, 5, 1, 8, 0), (63, 5, 1, 9, 0), (65, 9, 2, 4, 0), (12289, 9, 1, 6, 0), (49151, 120, 2, 4, 0), (49152, 120, 2, 4, 0),
+    (50000, 120, 3, 3, 0), (50000, 1200, 12, 6, 0), (50000, 1200, 13, 6, 0), (13000, 6, 30, 3, 150), (300, 6, 30, 3, 150),
     (32769, 6, 3, 3, 500), (12300, 6, 1, 3, 3000)])
 def test_margins_where_rows_take_few_or_uneven_steps(xgb, rows, cols, trees, depth, chain):
     """Both sides of the limits of the row-a-lane kernel: few steps a row, wide

@@ -421,15 +421,15 @@ __global__ __launch_bounds__(kDirectWaves * kWave) void k_predict_direct(Predict
 // deepest one's steps.  Whole calls, this kernel against the other, us:
 // - one tree of depth 6: 12,000 x 64 33 / 40, 1M x 8 493 / 510, CSR 200,000 x 2,000
 //   115 / 130, 64 rows 29 to 33 / 30 to 33; two: 1,000 x 64 33 / 32, 100,000 x 64 71 / 65;
-// - staged rows of many columns: 100,000 x 400, 24 steps 93 / 120, 48 131 / 131,
+// - staged rows of many columns: 100,000 x 400, 30 steps 92 / 126, 48 131 / 131,
 //   96 176 / 124; 1M x 128, 6 steps 593 / 681, 12 685 / 666 (13,000 x 400, 24: 42 / 41);
-// - rows too wide for LDS: 200,000 x 20,000 CSR, 48 steps 295 / 455, 96 431 / 372;
-//   100,000 x 1,200 138 / 179, 207 / 192 (13,000 x 1,200, 48: 61 / 46);
+// - rows too wide for LDS: 200,000 x 20,000 CSR, 60 steps 366 / 453, 96 431 / 372;
+//   200,000 x 1,200, 60 257 / 319 (33,000 x 1,200, 72: 86 / 72);
 // - one tree of depth 200 among 99 of depth 6 (20,000 steps for 794): 200,000 x 32
 //   676 / 1,685, 13,000 226 / 289; among nine (2,000 for 254) 276 / 287, 90 / 128.
 constexpr uint32_t kRowThreads = 64;
-constexpr uint32_t kRowsSteps = 8, kRowsFarSteps = 48, kRowsColumns = 14, kRowsDepths = 12;
-constexpr uint32_t kRowsMany = 32768;
+constexpr uint32_t kRowsSteps = 8, kRowsFarSteps = 72, kRowsColumns = 11, kRowsDepths = 12;
+constexpr uint32_t kRowsMany = 49152;
 template <bool SPARSE>
 __global__ __launch_bounds__(kRowThreads) void k_predict_rows(PredictArgs a) {
   for (uint64_t r = (uint64_t)blockIdx.x * kRowThreads + threadIdx.x; r < a.rows; r += (uint64_t)gridDim.x * kRowThreads) {
