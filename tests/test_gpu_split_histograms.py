@@ -50,3 +50,22 @@ def test_same_trees_over_options(xgb, extra):
     params = {"max_depth": 6, "max_bin": 128, **extra}
     _both(xgb, X, y, params, 4)
     _both(xgb, X, y, params, 4, weight=np.random.default_rng(1).uniform(0, 2, 7001).astype(np.float32))
+
+
+@pytest.mark.parametrize("rows,share", [(70000, 0.9), (80000, 0.9), (150000, 1.0), (600000, 0.95)])
+def test_csr_row_tiles_train_the_same_trees(xgb, rows, share):
+    """CSR row tiles are work units only: the default, which grows with a
+    column's entries (64 rows up to 65,536, 512 from 262,145 on), and given ones
+    train the same trees."""
+    import scipy.sparse as sp
+    rng = np.random.default_rng(rows)
+    dense = rng.normal(size=(rows, 3)).astype(np.float32)
+    dense[rng.random(dense.shape) > share] = 0
+    y = (dense[:, 0] * dense[:, 1] + 0.2 * rng.normal(size=rows)).astype(np.float32)
+    d = xgb.DMatrix(sp.csr_matrix(dense), label=y)
+    params = {"max_depth": 5, "max_bin": 64, "eta": 0.5}
+    models = []
+    for extra in ({}, {"hip_histogram_rows": 64}, {"hip_histogram_rows": 512}):
+        bst = xgb.train({**params, **extra}, d, 2)
+        models.append(json.loads(bst.save_raw("json"))["learner"]["gradient_booster"]["model"]["trees"])
+    assert models[0] == models[1] == models[2]

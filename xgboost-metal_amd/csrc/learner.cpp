@@ -907,12 +907,19 @@ void Learner::grow(DMatrix& data, bool unit_hessian, bool sampled) {
     // entries a row: some 10,000 rows a level), which tiles of 512 rows left to
     // twenty workgroups.  10 rounds at 64 / 128 / 256 / 512 rows: 1M x 2,000 15.1
     // / 15.1 / 16.0 / 18.2 ms, 100,000 x 2,000 7.9 / 8.4 / 9.3 / 11.3, 50,000 x
-    // 300 (10 a row) 3.0 / 3.2 / 3.5 / 4.3, 500,000 x 100 (24 a row) 27.7 / 27.5
-    // / 27.7 / 27.5.
+    // 300 (10 a row) 3.0 / 3.2 / 3.5 / 4.3.  Columns of many entries give the built
+    // child many rows, and so many tiles that their flushes and tasks cost more:
+    // the tile is doubled while a column holds over kTileEntries entries a row of
+    // it.  500,000 x 100 (24 a row, 120,000 a column) 5 rounds 16.0 / 15.8 / 15.8 /
+    // 15.7, 300,000 x 100 (50 a row, 150,000) 3 rounds 9.10 / 9.12 / 9.14 / 9.20, 2M x 40
+    // (10 a row, 500,000) 3 rounds 32.8 / 32.5 / 31.6 / 31.2.
+    constexpr uint64_t kTileEntries = 1024;
+    uint32_t tile = 64;
+    while (tile < 512 && data.values.size() / data.cols > kTileEntries * tile) tile *= 2;
     shape.sparse = 1;
     shape.compact_sampled = 0;
     shape.column_levels = 0;
-    shape.rows_per_tile = (uint32_t)integer("hip_histogram_rows", 64);
+    shape.rows_per_tile = (uint32_t)integer("hip_histogram_rows", tile);
     shape.root_rows_per_tile = 0;
   }
   size_t ws = mgb_tree_workspace_bytes(&shape);
