@@ -69,3 +69,10 @@ def test_csr_row_tiles_train_the_same_trees(xgb, rows, share):
         bst = xgb.train({**params, **extra}, d, 2)
         models.append(json.loads(bst.save_raw("json"))["learner"]["gradient_booster"]["model"]["trees"])
     assert models[0] == models[1] == models[2]
+
+
+@pytest.mark.parametrize("rows,cols", [(40960, 5), (40961, 5), (49153, 47), (49153, 48)])
+def test_same_trees_of_few_columns(xgb, rows, cols):
+    X, y = W.config1(rows=rows, cols=cols)
+    _both(xgb, X, y, {"max_depth": 5, "max_bin": 200}, 2)
+    _both(xgb, X, (y > 0).astype(np.float32), {"max_depth": 5, "max_bin": 200, "objective": "binary:logistic"}, 2)

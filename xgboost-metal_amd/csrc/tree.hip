@@ -3114,10 +3114,21 @@ int launch_split(const Tree& t, uint32_t depth, uint32_t items) {
 // (logistic) 15.1 -> 12.5, 32,000 x 32 depth 6 8.0 -> 7.2, 60,000 x 64 depth 8
 // 14.2 -> 13.4, 60,000 x 32 depth 6 8.5 -> 8.3 (every level: 8.4); beyond, the
 // gathered codes cost more than the launch: 100,000 x 32 depth 6 8.8 -> 9.1,
-// 262,144 x 64 16.6 -> 20.4.
+// 262,144 x 64 16.6 -> 20.4.  Many columns and two-byte codes gain more, their
+// codes' size notwithstanding (10 rounds, depth 6 or 8: 60,000 x 1,000 6.5 -> 5.6,
+// of 1,024 bins 16.4 -> 12.3, 65,000 x 600 8.9 -> 8.1); few columns of one-byte
+// codes, whose few items then are a level's whole work, lose at the large nodes
+// of many rows and take kOwnNodeFew there: depth 6, launches / nodes of at most
+// 16,384 / of 6,144, logistic, 65,536 rows x 3 1.82 / 1.96 / 1.81 ms, x 16 1.88 / 1.97 /
+// 1.86, x 31 1.98 / 2.00 / 1.93 (x 64 2.15 / 2.12), 60,000 x 8 1.87 / 1.95 / 1.86, 33,000
+// x 8 1.77 / 1.73 / 1.74, 16,000 x 16 1.81 / 1.62 / 1.66; squared error, 65,536 x 3 1.71
+// / 1.69 / 1.59.
 constexpr uint32_t kOwnRows = 65536, kOwnNode = 16384;
+constexpr uint32_t kOwnNodeFew = 6144, kOwnFewColumns = 48, kOwnFewRows = 40960;
 bool own_level(const Tree& t, uint32_t depth) {
-  return depth > 0 && t.columns && t.column_levels <= 1 && t.rows_n <= kOwnRows && (t.rows_n >> depth) <= kOwnNode;
+  const bool few = t.cols < kOwnFewColumns && t.bin_bytes == 1 && t.rows_n > kOwnFewRows;
+  return depth > 0 && t.columns && t.column_levels <= 1 && t.rows_n <= kOwnRows &&
+         (t.rows_n >> depth) <= (few ? kOwnNodeFew : kOwnNode);
 }
 
 // Select + partition of a level: `grid` partition workgroups plus the
