@@ -48,3 +48,22 @@ def test_large_uploads(nbytes):
         host_after = host.copy()
         host[:] = 0  # the copy is complete when the call returns
         np.testing.assert_array_equal(dev.read(np.uint8, nbytes), host_after)
+
+
+@pytest.mark.parametrize("rows,cols", [(1, 1), (7, 1), (1, 9), (13, 5), (1000, 17)])
+@pytest.mark.parametrize("dtype", ["float16", "float32", "float64", "int8", "uint16", "int32", "int64", "bool"])
+def test_layouts_and_types_keep_their_values(xgb, rows, cols, dtype):
+    """Every order and stride of every element type, 1-dimensional labels among
+    them."""
+    rng = np.random.default_rng(rows * 31 + cols)
+    plain = rng.integers(0, 2 if dtype == "bool" else 100, size=(rows, cols)).astype(dtype)
+    wide = np.zeros((2 * rows, 3 * cols), dtype)
+    wide[::2, ::3] = plain
+    want = plain.astype(np.float32)
+    for given in (plain, np.asfortranarray(plain), wide[::2, ::3], plain[::-1, ::-1][::-1, ::-1], wide[::2, ::3][::-1][::-1]):
+        got = xgb.DMatrix(given).get_data()
+        np.testing.assert_array_equal(got.toarray(), want)
+    reverse = xgb.DMatrix(plain[::-1, ::-1]).get_data()
+    np.testing.assert_array_equal(reverse.toarray(), want[::-1, ::-1])
+    labelled = xgb.DMatrix(plain, label=wide[::2, 0])
+    np.testing.assert_array_equal(labelled.get_label(), want[:, 0])

@@ -165,14 +165,23 @@ HostFloats to_vector(const ArrayView& v) {
     copy_large(out.data(), v.data, (size_t)n * sizeof(float));
     return out;
   }
-  if (v.shape.size() == 1) {
-    for (int64_t i = 0; i < n; ++i) out[i] = load_value(v, i * v.strides[0]);
-  } else if (v.shape.size() == 2) {
-    int64_t cols = v.shape[1];
-    for (int64_t r = 0; r < v.shape[0]; ++r)
-      for (int64_t c = 0; c < cols; ++c) out[r * cols + c] = load_value(v, r * v.strides[0] + c * v.strides[1]);
+  require(v.shape.size() == 1 || v.shape.size() == 2, "Only 1- and 2-dimensional arrays are supported.");
+  const int64_t rows = v.shape[0], cols = v.shape.size() == 2 ? v.shape[1] : 1;
+  const int64_t row_step = v.strides[0], col_step = v.shape.size() == 2 ? v.strides[1] : 0;
+  float* dst = out.data();
+  auto gather = [&](auto value) {
+    for (int64_t r = 0; r < rows; ++r)
+      for (int64_t c = 0; c < cols; ++c) *dst++ = value(r * row_step + c * col_step);
+  };
+  if (v.kind == 'f' && v.itemsize == 4) {
+    const uint8_t* data = v.data;
+    gather([data](int64_t offset) {
+      float f;
+      std::memcpy(&f, data + offset, sizeof(f));
+      return f;
+    });
   } else {
-    throw Error("Only 1- and 2-dimensional arrays are supported.");
+    gather([&v](int64_t offset) { return load_value(v, offset); });
   }
   return out;
 }

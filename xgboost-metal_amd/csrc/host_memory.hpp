@@ -59,7 +59,8 @@ using HostFloats = std::vector<float, HostAllocator<float>>;
 // leaves its share to the caller.
 inline void copy_large(void* dst, const void* src, size_t bytes) {
   constexpr size_t kShare = size_t(4) << 20;
-  const size_t n = std::min({bytes / kShare, size_t(8), (size_t)std::max(1u, std::thread::hardware_concurrency())});
+  size_t n = std::min(bytes / kShare, size_t(8));
+  if (n > 1) n = std::min(n, (size_t)std::max(1u, std::thread::hardware_concurrency()));  // a system call
   if (n <= 1) {
     if (bytes) std::memcpy(dst, src, bytes);
     return;
