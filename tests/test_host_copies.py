@@ -67,3 +67,25 @@ def test_layouts_and_types_keep_their_values(xgb, rows, cols, dtype):
     np.testing.assert_array_equal(reverse.toarray(), want[::-1, ::-1])
     labelled = xgb.DMatrix(plain, label=wide[::2, 0])
     np.testing.assert_array_equal(labelled.get_label(), want[:, 0])
+
+
+@pytest.mark.parametrize("kind", ["csr", "csc", "coo"])
+def test_sparse_offsets_and_columns_past_2_24(xgb, kind):
+    """Offsets and indices that binary32 does not hold."""
+    import scipy.sparse as sp
+    n = (1 << 24) + 1
+    if kind == "csr":
+        # Row 0 is column 0's .. 2^24's, row 1 one entry behind them.
+        m = sp.csr_matrix((np.ones(n + 1, np.float32), np.append(np.arange(n), n).astype(np.int64),
+                           np.array([0, n, n + 1], np.int64)), shape=(2, n + 2))
+    elif kind == "csc":
+        m = sp.csc_matrix((np.ones(n + 1, np.float32), np.append(np.arange(n), n).astype(np.int64),
+                           np.array([0, n, n + 1], np.int64)), shape=(n + 2, 2))
+    else:
+        m = sp.coo_matrix((np.array([3.0, 4.0], np.float32), (np.array([n, 5]), np.array([1, n]))), shape=(n + 2, n + 2))
+    got = xgb.DMatrix(m).get_data()
+    want = m.tocsr()
+    assert got.shape == want.shape
+    np.testing.assert_array_equal(got.indptr, want.indptr)
+    np.testing.assert_array_equal(got.indices, want.indices)
+    np.testing.assert_array_equal(got.data, want.data)

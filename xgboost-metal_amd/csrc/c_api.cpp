@@ -150,6 +150,21 @@ float load_value(const ArrayView& v, int64_t offset) {
   throw Error("Unsupported array dtype.");
 }
 
+// Offsets and indices: whole numbers past 2^24 are not binary32 values.
+int64_t load_index(const ArrayView& v, int64_t offset) {
+  const uint8_t* p = v.data + offset;
+  auto whole = [p](auto x) {
+    std::memcpy(&x, p, sizeof(x));
+    return (int64_t)x;
+  };
+  if (v.kind == 'i' && v.itemsize == 4) return whole(int32_t{});
+  if (v.kind == 'i' && v.itemsize == 8) return whole(int64_t{});
+  if (v.kind == 'u' && v.itemsize == 4) return whole(uint32_t{});
+  if (v.kind == 'u' && v.itemsize == 8) return whole(uint64_t{});
+  if (v.kind == 'f' && v.itemsize == 8) return whole(double{});
+  return (int64_t)load_value(v, offset);
+}
+
 HostFloats to_vector(const ArrayView& v) {
   int64_t n = 1;
   for (auto d : v.shape) n *= d;
@@ -306,12 +321,12 @@ std::shared_ptr<DMatrix> csr_from_interfaces(const char* indptr, const char* ind
   const int64_t rows = ip.shape[0] - 1;
   require(rows >= 0, "Invalid CSR indptr.");
   return csr_matrix((uint64_t)rows, ncol, missing, [&](uint64_t r, std::vector<std::pair<uint32_t, float>>& row) {
-    const int64_t b = (int64_t)load_value(ip, (int64_t)r * ip.strides[0]);
-    const int64_t e = (int64_t)load_value(ip, (int64_t)(r + 1) * ip.strides[0]);
+    const int64_t b = load_index(ip, (int64_t)r * ip.strides[0]);
+    const int64_t e = load_index(ip, (int64_t)(r + 1) * ip.strides[0]);
     require(b >= 0 && e >= b && e <= ix.shape[0] && e <= dv.shape[0], "Invalid CSR indptr.");
     for (int64_t k = b; k < e; ++k) {
-      const int64_t c = (int64_t)load_value(ix, k * ix.strides[0]);
-      require(c >= 0, "CSR column index out of range.");
+      const int64_t c = load_index(ix, k * ix.strides[0]);
+      require(c >= 0 && c <= (int64_t)UINT32_MAX, "CSR column index out of range.");
       row.emplace_back((uint32_t)c, load_value(dv, k * dv.strides[0]));
     }
   });
@@ -1125,10 +1140,10 @@ int XGDMatrixCreateFromCSC(char const* indptr, char const* indices, char const* 
   // Column order: each row receives its entries with increasing columns.
   std::vector<std::vector<std::pair<uint32_t, float>>> rows((size_t)nrow);
   for (int64_t c = 0; c < ncol; ++c) {
-    const int64_t b = (int64_t)load_value(cp, c * cp.strides[0]), e = (int64_t)load_value(cp, (c + 1) * cp.strides[0]);
+    const int64_t b = load_index(cp, c * cp.strides[0]), e = load_index(cp, (c + 1) * cp.strides[0]);
     require(b >= 0 && e >= b && e <= ri.shape[0] && e <= dv.shape[0], "Invalid CSC indptr.");
     for (int64_t k = b; k < e; ++k) {
-      const int64_t r = (int64_t)load_value(ri, k * ri.strides[0]);
+      const int64_t r = load_index(ri, k * ri.strides[0]);
       require(r >= 0 && (uint64_t)r < nrow, "CSC row index out of range.");
       rows[(size_t)r].emplace_back((uint32_t)c, load_value(dv, k * dv.strides[0]));
     }
@@ -1148,7 +1163,7 @@ int XGDMatrixCreateFromCOO(char const* row_idx, char const* col_idx, char const*
   require(ri.shape[0] == ci.shape[0] && ri.shape[0] == dv.shape[0], "COO arrays differ in length.");
   std::vector<std::vector<std::pair<uint32_t, float>>> rows((size_t)nrow);
   for (int64_t k = 0; k < ri.shape[0]; ++k) {
-    const int64_t r = (int64_t)load_value(ri, k * ri.strides[0]), c = (int64_t)load_value(ci, k * ci.strides[0]);
+    const int64_t r = load_index(ri, k * ri.strides[0]), c = load_index(ci, k * ci.strides[0]);
     require(r >= 0 && (uint64_t)r < nrow && c >= 0 && (uint64_t)c < ncol, "COO index out of range.");
     rows[(size_t)r].emplace_back((uint32_t)c, load_value(dv, k * dv.strides[0]));
   }
