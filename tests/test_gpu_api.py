@@ -251,3 +251,27 @@ def test_device_status_refuses_round_and_rolls_back(xgb):
     assert bst.num_boosted_rounds() == 4
     assert _trees(bst) == _trees(clean4)
     np.testing.assert_array_equal(bst.predict(d).view(np.uint32), clean4.predict(d).view(np.uint32))
+
+
+def test_labels_set_after_a_fit_are_trained_on(xgb):
+    """New labels of a matrix that is binned already reach the device."""
+    rng = np.random.default_rng(11)
+    X = rng.normal(size=(3000, 5)).astype(np.float32)
+    first, second = X[:, 0].copy(), (X[:, 1] > 0).astype(np.float32)
+    for maker in (xgb.DMatrix, xgb.QuantileDMatrix):
+        d = maker(X, label=first)
+        xgb.train({"max_depth": 3}, d, 2)
+        d.set_label(second)
+        for params in ({"max_depth": 3}, {"max_depth": 3, "objective": "binary:logistic"}):
+            got = xgb.train(params, d, 3).predict(d)
+            np.testing.assert_array_equal(got, xgb.train(params, maker(X, label=second), 3).predict(xgb.DMatrix(X)))
+        # Between two rounds of one booster.
+        bst = xgb.Booster({"max_depth": 3}, [d])
+        bst.update(d, 0)
+        before = bst.predict(d, output_margin=True)
+        d.set_label(first)
+        bst.update(d, 1)
+        fresh = xgb.DMatrix(X, label=first, base_margin=before)
+        step = xgb.train({"max_depth": 3, "base_score": 0.0}, fresh, 1)
+        np.testing.assert_allclose(bst.predict(d, output_margin=True), step.predict(fresh, output_margin=True), rtol=0,
+                                   atol=1e-6)

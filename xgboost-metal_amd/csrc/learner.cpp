@@ -1093,6 +1093,7 @@ void Learner::update(DMatrix& data, int /*iteration*/) {
     require(labels_in_unit(data), "label must be in [0,1] for logistic loss.");
   }
   data.quantize((uint32_t)integer("max_bin", 256), bin_layout(), (uint32_t)integer("hip_histogram_features", 0));
+  data.upload_info();  // labels set since the matrix was binned
   auto t0 = std::chrono::steady_clock::now();
   initialize(data, false);
   if (data.rows == 0) return empty_round();
