@@ -455,7 +455,7 @@ struct ShapArgs {
 // (IN_LDS), where each wave has its own sums, added in wave order at the end;
 // more features than that holds keep both in memory, a partial to each wave.
 // Bound by vector operations, about 3 Q + 12 an element, and the chain of each
-// leaf's LDS sums.  5,000 x 32, 100 trees of depth 6: 0.137 ms, against 131.7
+// leaf's LDS sums.  5,000 x 32, 100 trees of depth 6: 0.13 ms, against 131.7
 // with a row a lane and the paths in scratch memory (LDS float atomics in the
 // place of load, add, store: 0.95 ms).  In memory, whole calls against a row a
 // lane, 100 trees of depth 8: 1 row x 2,000 0.51 against 297 ms, 5,000 rows 21.8

@@ -149,9 +149,8 @@ __device__ __forceinline__ void walk_some(uint32_t n, const StagedNodes& nodes, 
 // LDS and are added in tree order.  Measured against a row a lane with nodes
 // and values read from memory: 1M x 64, 100 trees of depth 8, 11.66 -> 0.65 ms
 // (0.10 of it the read of X); 100,003 x 32, depth 6, 440 -> 44 us; CSR 200,000
-// x 2,000 with 20 entries a row, 1.84 -> 0.21 ms (a search in the row at each
-// node before).  One 8-byte LDS read of a whole node costs more than two
-// 4-byte ones (13.6 cycles against 4 each at random addresses).
+// x 2,000 with 20 entries a row, 1.84 -> 0.22 ms (a search in the row at each
+// node before).  Words and links lie apart: two 4-byte LDS reads.
 template <bool SPARSE>
 __global__ __launch_bounds__(kStageWaves * kWave) void k_predict_staged(PredictArgs a) {
   extern __shared__ __align__(16) uint8_t p_smem[];

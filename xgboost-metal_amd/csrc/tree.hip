@@ -1607,7 +1607,10 @@ __device__ __forceinline__ void score_pair(NodeEval& na, const LaneBins<CH>& la,
 // four consecutive bins, whose in-lane prefix sums follow.  Loads of a lane's
 // four consecutive bins touch every line four times over: 1M x 2,000 CSR 107.9 ->
 // 94.9 us a launch at the wide levels, 262,144 x 64 25.5 -> 22.1, 1.5M x 128 at
-// 1,024 bins (four waves an item) 191 -> 185.
+// 1,024 bins (four waves an item) 191 -> 185.  An item of 16 waves (over 2,048
+// bins) has 82 KB of cells, which leaves a CU one workgroup, and still gains: fits
+// of 4,096 bins, 200,000 x 16, depth 6, 10 rounds 6.2 -> 4.6 ms, x 64, depth 8, 5
+// rounds 10.3 -> 7.9.
 constexpr uint32_t kStripePitch = 5;  // 16-byte cells of a lane's four bins, one more for the banks
 struct StripeCells {
   uint4 cell[kWave * kStripePitch];
