@@ -1368,7 +1368,7 @@ std::function<double(const double*)> Learner::metric(DMatrix& d, const float* pr
   if (it->second >= 13) {
     require(labels_in_unit(d), "AUC labels must be in [0,1].");
     if (!d.rows) return [nan](const double*) { return nan; };
-    if (auc_rows_ != d.rows) {
+    if (auc_rows_ != d.rows || !auc_bytes_) {  // 0: the query failed, and is asked again
       auc_bytes_ = mgb_metric_workspace_bytes(d.rows);
       auc_rows_ = d.rows;
     }
