@@ -3125,7 +3125,9 @@ int launch_split(const Tree& t, uint32_t depth, uint32_t items) {
 // 16,384 / of 6,144, logistic, 65,536 rows x 3 1.82 / 1.96 / 1.81 ms, x 16 1.88 / 1.97 /
 // 1.86, x 31 1.98 / 2.00 / 1.93 (x 64 2.15 / 2.12), 60,000 x 8 1.87 / 1.95 / 1.86, 33,000
 // x 8 1.77 / 1.73 / 1.74, 16,000 x 16 1.81 / 1.62 / 1.66; squared error, 65,536 x 3 1.71
-// / 1.69 / 1.59.
+// / 1.69 / 1.59.  The average is what the host knows: where thin tails are split
+// off first and a deep level halves one node of most rows, an item walks them
+// alone (65,000 x 200 made so 2.86 -> 3.08; where tails alone are split, 2.80 -> 2.39).
 constexpr uint32_t kOwnRows = 65536, kOwnNode = 16384;
 constexpr uint32_t kOwnNodeFew = 6144, kOwnFewColumns = 48, kOwnFewRows = 40960;
 bool own_level(const Tree& t, uint32_t depth) {
